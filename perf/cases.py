@@ -297,7 +297,7 @@ def tolerance(case):
     an append copies bits."""
     if case["kind"] == "append":
         return "exact"
-    return {"rel": BF16_TOL, "max": 0.1}
+    return {"rel": BF16_TOL, "max": 0.06}
 
 
 # ---------------------------------------------------------------------------
