@@ -178,14 +178,16 @@ gqa_decode_kernel(
   const Plan plan =
       plan_build<NT>(p.len_in, add, p.cap, p.B, p.Hkv, p.n_splits, s_pref, s_scan, s_len,
                      s_wpref, uniform(blockIdx.x * W + (tid >> 6)));
-  if (blockIdx.x == 0) {  // sequences without tokens: the empty partial (0, -inf),
-    for (int b = 0; b < p.B; ++b) {  // or NaN for an invalid length
-      if (s_pref[b + 1] != s_pref[b]) continue;
-      const bool ok = len_ok(p.len_in[b], add, p.cap);
-      const size_t q0 = (size_t)b * p.Hkv * GG;
-      for (int idx = tid; idx < p.Hkv * GG * D; idx += NT) p.out[q0 * D + idx] = ok ? 0.f : qnan();
-      for (int idx = tid; idx < p.Hkv * GG; idx += NT) p.lse[q0 + idx] = ok ? neg_inf() : qnan();
-    }
+  // Sequences without tokens: the empty partial (0, -inf), or NaN for an
+  // invalid length.  Workgroup g looks at sequences g, g + grid, ...: one
+  // workgroup looking at all of them is a chain of an LDS read per sequence
+  // (10 us at B = 256) ahead of its own blocks.
+  for (int b = blockIdx.x; b < p.B; b += gridDim.x) {
+    if (s_pref[b + 1] != s_pref[b]) continue;
+    const bool ok = len_ok(p.len_in[b], add, p.cap);
+    const size_t q0 = (size_t)b * p.Hkv * GG;
+    for (int idx = tid; idx < p.Hkv * GG * D; idx += NT) p.out[q0 * D + idx] = ok ? 0.f : qnan();
+    for (int idx = tid; idx < p.Hkv * GG; idx += NT) p.lse[q0 + idx] = ok ? neg_inf() : qnan();
   }
   const int split = uniform(blockIdx.x * W + (tid >> 6));
   if (!plan.has_work) return;  // no barrier below: waves run independently

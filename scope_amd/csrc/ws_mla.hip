@@ -125,14 +125,14 @@ __global__ __launch_bounds__(256) void mla_decode_kernel(const MlaParams p) {
       p.len_out[b] = step_len_out(p.len_in, b, add, p.cap);
   const Plan plan = plan_build<NT>(p.len_in, add, p.cap, p.B, 1, gridDim.x, s_pref, s_scan,
                                    s_len, s_wpref, g, p.ng);
-  if (g == 0) {  // sequences without tokens: the empty partial (0, -inf), or
-    for (int b = 0; b < p.B; ++b) {  // NaN for an invalid length
-      if (s_pref[b + 1] != s_pref[b]) continue;
-      const bool ok = len_ok(p.len_in[seq_of(b, p.ng)], add, p.cap);
-      for (int idx = tid; idx < kMlaH * kMlaC; idx += NT)
-        p.out[(size_t)b * kMlaH * kMlaC + idx] = ok ? 0.f : qnan();
-      if (tid < kMlaH) p.lse[b * kMlaH + tid] = ok ? neg_inf() : qnan();
-    }
+  // sequences without tokens: the empty partial (0, -inf), or NaN for an
+  // invalid length (spread over the workgroups, as in gqa_decode_kernel)
+  for (int b = g; b < p.B; b += gridDim.x) {
+    if (s_pref[b + 1] != s_pref[b]) continue;
+    const bool ok = len_ok(p.len_in[seq_of(b, p.ng)], add, p.cap);
+    for (int idx = tid; idx < kMlaH * kMlaC; idx += NT)
+      p.out[(size_t)b * kMlaH * kMlaC + idx] = ok ? 0.f : qnan();
+    if (tid < kMlaH) p.lse[b * kMlaH + tid] = ok ? neg_inf() : qnan();
   }
   if (!plan.has_work) return;
   const int blk_begin = uniform(plan.begin);  // (the compiler cannot tell on its own)
