@@ -114,6 +114,11 @@ struct MergeSplitParams {
   float* lse_out;
 };
 
+// LDS of a merge: one weight per piece a row can have (a row's pieces come from
+// different splits).  Sized by the call, not by the most a call may have: 16
+// KB kept a CU to nine of these one-wave workgroups.
+static size_t merge_lds(int n) { return 4 * (size_t)n; }
+
 // One 64-lane workgroup per (output row, 256-column chunk): lane t owns float4
 // column chunk * 64 + t and accumulates it over the pieces with eight loads
 // in flight.
@@ -121,10 +126,7 @@ constexpr int kMergeChunk4 = 64;
 
 template <int FMT>
 __global__ __launch_bounds__(64) void merge_split_kernel(const MergeSplitParams p) {
-  __shared__ int s_pref[kMaxSeqs + 1];
-  __shared__ int s_wpref[kSeqPlanMax + 1];
-  __shared__ int s_scan[2];
-  __shared__ float s_w[kReduceMaxWeights];
+  extern __shared__ float s_w[];  // weights of the row's pieces (at most p.grid)
   const int qrow = blockIdx.x;
   const int t = threadIdx.x;
   const int krow = qrow / p.heads;
@@ -140,9 +142,7 @@ __global__ __launch_bounds__(64) void merge_split_kernel(const MergeSplitParams 
   if (FMT >= 0)
     load_b<(FMT >= 0 ? FMT : 0)>(p.b_out, p.b_aux0, p.b_aux1, qrow, p.Dv, col_ok ? c : 0, lb,
                                  ob);
-  const Plan plan = plan_build<64>(p.gpu_len, p.add, p.cap, p.B, p.R, p.grid, s_pref, s_scan,
-                                   nullptr, s_wpref, -1, p.ng);
-  const int nbb = (plan_len(p.gpu_len, seq_of(b, p.ng), p.add, p.cap) + 31) >> 5;
+  const RowSplits rs = plan_row(p.gpu_len, p.add, p.cap, p.B, p.R, p.grid, b, r, p.ng);
   // One piece: the step's final partial (out_g, fp32); several: their bf16
   // workspace slots, piece s at pieces + s * sstride.
   int n = 1;
@@ -150,18 +150,13 @@ __global__ __launch_bounds__(64) void merge_split_kernel(const MergeSplitParams 
   const uint16_t* pieces = nullptr;
   const float* lsrc = p.lse_g + qrow;  // lse of piece s at lsrc[s * lstride]
   size_t sstride = 0, lstride = 0;
-  if (nbb > 0 && plan.n > 0) {
-    const int row_start = s_pref[b] + r * nbb;
-    int w_first, nseg;
-    plan_row_splits(plan, b, row_start, nbb, s_wpref, w_first, nseg);
-    if (nseg > 1) {
-      n = nseg;
-      const size_t slot0 = (size_t)(w_first + krow) * p.heads + h;
-      pieces = p.part_out + slot0 * p.Dv;
-      lsrc = p.part_lse + slot0;
-      sstride = (size_t)p.heads * p.Dv;
-      lstride = p.heads;
-    }
+  if (rs.nseg > 1) {
+    n = rs.nseg;
+    const size_t slot0 = (size_t)(rs.w_first + krow) * p.heads + h;
+    pieces = p.part_out + slot0 * p.Dv;
+    lsrc = p.part_lse + slot0;
+    sstride = (size_t)p.heads * p.Dv;
+    lstride = p.heads;
   }
   // The pieces' columns are requested with their lse values.
   const int cc = col_ok ? c : 0;
@@ -234,10 +229,7 @@ template <int FMT>
 __global__ __launch_bounds__(kUvThreads) void merge_split_uv_kernel(
     const MergeSplitParams p, const uint16_t* __restrict__ w_uv, int Dout,
     uint16_t* __restrict__ out_v) {
-  __shared__ int s_pref[kMaxSeqs + 1];
-  __shared__ int s_wpref[kSeqPlanMax + 1];
-  __shared__ int s_scan[kUvThreads / 64 + 1];
-  __shared__ float s_w[kReduceMaxWeights];
+  extern __shared__ float s_w[];  // weights of the row's pieces (at most p.grid)
   __shared__ float s_row[512];
   __shared__ float s_ml[2];  // M, 1 / L
   const int qrow = blockIdx.x;  // b * heads + h
@@ -266,27 +258,19 @@ __global__ __launch_bounds__(kUvThreads) void merge_split_uv_kernel(
   float4 ob = make_float4(0.f, 0.f, 0.f, 0.f);
   if (FMT >= 0 && merging)
     load_b<(FMT >= 0 ? FMT : 0)>(p.b_out, p.b_aux0, p.b_aux1, qrow, p.Dv, c, lb, ob);
-  const Plan plan =
-      plan_build<kUvThreads>(p.gpu_len, p.add, p.cap, p.B, 1, p.grid, s_pref, s_scan, nullptr,
-                             s_wpref, -1, p.ng);
-  const int nbb = (plan_len(p.gpu_len, b, p.add, p.cap) + 31) >> 5;
+  const RowSplits rs = plan_row(p.gpu_len, p.add, p.cap, p.B, 1, p.grid, pv_seq, 0, p.ng);
   int n = 1;
   const float* src = p.out_g + (size_t)qrow * p.Dv;
   const uint16_t* pieces = nullptr;
   const float* lsrc = p.lse_g + qrow;
   size_t sstride = 0, lstride = 0;
-  if (nbb > 0 && plan.n > 0) {
-    const int row_start = s_pref[pv_seq];
-    int w_first, nseg;
-    plan_row_splits(plan, pv_seq, row_start, nbb, s_wpref, w_first, nseg);
-    if (nseg > 1) {  // pieces hold hp heads each
-      n = nseg;
-      const size_t slot0 = (size_t)(w_first + pv_seq) * hp + h16;
-      pieces = p.part_out + slot0 * p.Dv;
-      lsrc = p.part_lse + slot0;
-      sstride = (size_t)hp * p.Dv;
-      lstride = hp;
-    }
+  if (rs.nseg > 1) {  // pieces hold hp heads each
+    n = rs.nseg;
+    const size_t slot0 = (size_t)(rs.w_first + pv_seq) * hp + h16;
+    pieces = p.part_out + slot0 * p.Dv;
+    lsrc = p.part_lse + slot0;
+    sstride = (size_t)hp * p.Dv;
+    lstride = hp;
   }
   // The merging threads' piece columns are requested with the lse values.
   uint2 pv[8];
@@ -412,8 +396,8 @@ int merge_split_pieces(const int32_t* len, int len_add, int B, int R, int heads,
   prm.out_bf16 = out_bf16;
   prm.out_f32 = out;
   prm.lse_out = lse;
-  hipLaunchKernelGGL(merge_split_kernel<-1>, dim3((unsigned)(B * R * heads)), dim3(64), 0,
-                     stream, prm);
+  hipLaunchKernelGGL(merge_split_kernel<-1>, dim3((unsigned)(B * R * heads)), dim3(64),
+                     merge_lds(n), stream, prm);
   return WS_OK;
 }
 
@@ -493,23 +477,28 @@ extern "C" int ws_merge_split(const int32_t* gpu_len, int B, int rows_per_seq, i
   const dim3 block(64);
   hipStream_t s = (hipStream_t)stream;
   if (!b_out) {
-    hipLaunchKernelGGL(merge_split_kernel<-1>, grid, block, 0, s, prm);
+    hipLaunchKernelGGL(merge_split_kernel<-1>, grid, block, merge_lds(n_workgroups), s, prm);
   } else {
     switch (fmt_b) {
       case WS_PARTIAL_LSE_F32:
-        hipLaunchKernelGGL(merge_split_kernel<WS_PARTIAL_LSE_F32>, grid, block, 0, s, prm);
+        hipLaunchKernelGGL(merge_split_kernel<WS_PARTIAL_LSE_F32>, grid, block, merge_lds(n_workgroups),
+                           s, prm);
         break;
       case WS_TRIPLE_UNNORM_F32:
-        hipLaunchKernelGGL(merge_split_kernel<WS_TRIPLE_UNNORM_F32>, grid, block, 0, s, prm);
+        hipLaunchKernelGGL(merge_split_kernel<WS_TRIPLE_UNNORM_F32>, grid, block, merge_lds(n_workgroups),
+                           s, prm);
         break;
       case WS_TRIPLE_NORM_BF16:
-        hipLaunchKernelGGL(merge_split_kernel<WS_TRIPLE_NORM_BF16>, grid, block, 0, s, prm);
+        hipLaunchKernelGGL(merge_split_kernel<WS_TRIPLE_NORM_BF16>, grid, block, merge_lds(n_workgroups),
+                           s, prm);
         break;
       case WS_PARTIAL_LSE_BF16:
-        hipLaunchKernelGGL(merge_split_kernel<WS_PARTIAL_LSE_BF16>, grid, block, 0, s, prm);
+        hipLaunchKernelGGL(merge_split_kernel<WS_PARTIAL_LSE_BF16>, grid, block, merge_lds(n_workgroups),
+                           s, prm);
         break;
       default:
-        hipLaunchKernelGGL(merge_split_kernel<WS_TRIPLE_NORM_F32>, grid, block, 0, s, prm);
+        hipLaunchKernelGGL(merge_split_kernel<WS_TRIPLE_NORM_F32>, grid, block, merge_lds(n_workgroups),
+                           s, prm);
         break;
     }
   }
@@ -613,28 +602,29 @@ extern "C" int ws_mla_merge_split_uv(const int32_t* gpu_len, int B, int heads,
   const dim3 block(kUvThreads);
   hipStream_t s = (hipStream_t)stream;
   if (!b_out) {
-    hipLaunchKernelGGL(merge_split_uv_kernel<-1>, grid, block, 0, s, prm, w_uv, Dout, out_v);
+    hipLaunchKernelGGL(merge_split_uv_kernel<-1>, grid, block, merge_lds(n_workgroups), s, prm, w_uv,
+                       Dout, out_v);
   } else {
     switch (fmt_b) {
       case WS_PARTIAL_LSE_F32:
-        hipLaunchKernelGGL(merge_split_uv_kernel<WS_PARTIAL_LSE_F32>, grid, block, 0, s, prm,
-                           w_uv, Dout, out_v);
+        hipLaunchKernelGGL(merge_split_uv_kernel<WS_PARTIAL_LSE_F32>, grid, block, merge_lds(n_workgroups), s,
+                           prm, w_uv, Dout, out_v);
         break;
       case WS_TRIPLE_UNNORM_F32:
-        hipLaunchKernelGGL(merge_split_uv_kernel<WS_TRIPLE_UNNORM_F32>, grid, block, 0, s, prm,
-                           w_uv, Dout, out_v);
+        hipLaunchKernelGGL(merge_split_uv_kernel<WS_TRIPLE_UNNORM_F32>, grid, block, merge_lds(n_workgroups), s,
+                           prm, w_uv, Dout, out_v);
         break;
       case WS_TRIPLE_NORM_BF16:
-        hipLaunchKernelGGL(merge_split_uv_kernel<WS_TRIPLE_NORM_BF16>, grid, block, 0, s, prm,
-                           w_uv, Dout, out_v);
+        hipLaunchKernelGGL(merge_split_uv_kernel<WS_TRIPLE_NORM_BF16>, grid, block, merge_lds(n_workgroups), s,
+                           prm, w_uv, Dout, out_v);
         break;
       case WS_PARTIAL_LSE_BF16:
-        hipLaunchKernelGGL(merge_split_uv_kernel<WS_PARTIAL_LSE_BF16>, grid, block, 0, s, prm,
-                           w_uv, Dout, out_v);
+        hipLaunchKernelGGL(merge_split_uv_kernel<WS_PARTIAL_LSE_BF16>, grid, block, merge_lds(n_workgroups), s,
+                           prm, w_uv, Dout, out_v);
         break;
       default:
-        hipLaunchKernelGGL(merge_split_uv_kernel<WS_TRIPLE_NORM_F32>, grid, block, 0, s, prm,
-                           w_uv, Dout, out_v);
+        hipLaunchKernelGGL(merge_split_uv_kernel<WS_TRIPLE_NORM_F32>, grid, block, merge_lds(n_workgroups), s,
+                           prm, w_uv, Dout, out_v);
         break;
     }
   }

@@ -104,7 +104,6 @@ __global__ __launch_bounds__(256) void mla_decode_kernel(const MlaParams p) {
   __shared__ int s_pref[kMaxSeqs + 1];
   __shared__ int s_len[kMaxSeqs];
   __shared__ int s_wpref[kSeqPlanMax + 1];
-  __shared__ int s_scan[NT / 64 + 1];
   const int g = blockIdx.x;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -123,8 +122,8 @@ __global__ __launch_bounds__(256) void mla_decode_kernel(const MlaParams p) {
   if (APPEND && p.len_out && g == 0)
     for (int b = tid; b < p.B / p.ng; b += NT)
       p.len_out[b] = step_len_out(p.len_in, b, add, p.cap);
-  const Plan plan = plan_build<NT>(p.len_in, add, p.cap, p.B, 1, gridDim.x, s_pref, s_scan,
-                                   s_len, s_wpref, g, p.ng);
+  const Plan plan = plan_build(p.len_in, add, p.cap, p.B, 1, gridDim.x, s_pref, s_len, s_wpref, g,
+                               p.ng);
   // sequences without tokens: the empty partial (0, -inf), or NaN for an
   // invalid length (spread over the workgroups, as in gqa_decode_kernel)
   for (int b = g; b < p.B; b += gridDim.x) {
@@ -141,8 +140,7 @@ __global__ __launch_bounds__(256) void mla_decode_kernel(const MlaParams p) {
   const u32x4* dummy = (const u32x4*)p.q_nope;
 
   while (blk < blk_end) {
-    const int b = uniform((blk == blk_begin && plan.b0 >= 0) ? plan.b0
-                                                             : plan_seq(s_pref, p.B, blk));
+    const int b = uniform(blk == blk_begin ? plan.b0 : plan_seq(s_pref, p.B, blk));
     const int len = uniform(s_len[b]);
     const int len_old = len - add;
     const int row_start = uniform(s_pref[b]);
@@ -418,24 +416,17 @@ namespace ws {
 // Runs after the decode kernel on the same stream, so plain loads see the
 // partials.
 __global__ __launch_bounds__(64) void mla_reduce_kernel(const MlaParams p, int grid) {
-  __shared__ int s_pref[kMaxSeqs + 1];
-  __shared__ int s_wpref[kSeqPlanMax + 1];
-  __shared__ int s_scan[2];
-  __shared__ float s_w[kReduceMaxWeights];
+  extern __shared__ float s_w[];  // weights of the row's pieces (at most grid)
   const int hrow = blockIdx.x;  // b * hp + h
   const int chunk = blockIdx.y;
   const int t = threadIdx.x;
   const int b = hrow / p.hp;
   const int h = hrow - b * p.hp;
   const int add = p.c_new ? 1 : 0;
-  const Plan plan = plan_build<64>(p.len_in, add, p.cap, p.B, 1, grid, s_pref, s_scan, nullptr,
-                                   s_wpref, -1, p.ng);
-  const int row_start = s_pref[b], row_end = s_pref[b + 1];
-  if (row_end == row_start) return;
-  int w_first, n;
-  plan_row_splits(plan, b, row_start, row_end - row_start, s_wpref, w_first, n);
-  if (n == 1) return;
-  const size_t slot0 = (size_t)(w_first + b) * p.hp + h;  // partial row of split 0
+  const RowSplits rs = plan_row(p.len_in, add, p.cap, p.B, 1, grid, b, 0, p.ng);
+  const int n = rs.nseg;
+  if (n <= 1) return;
+  const size_t slot0 = (size_t)(rs.w_first + b) * p.hp + h;  // partial row of split 0
   const int c = chunk * 64 + t;  // float4 column
   // the pieces' columns are requested with their lse values
   uint2 pv[8];
@@ -568,7 +559,8 @@ static int mla_launch(const uint16_t* q_nope, const uint16_t* q_pe,
   }
   int rc = check_launch(name);
   if (rc || n == 1 || !combine) return rc;
-  hipLaunchKernelGGL(mla_reduce_kernel, dim3(Bv * hp, kMlaC / 256), dim3(64), 0, s, prm, n);
+  hipLaunchKernelGGL(mla_reduce_kernel, dim3(Bv * hp, kMlaC / 256), dim3(64),
+                     4 * (size_t)n, s, prm, n);
   return check_launch(name);
 }
 

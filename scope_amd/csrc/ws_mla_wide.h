@@ -193,7 +193,6 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
   __shared__ int s_pref[kWideMaxSeqs + 1];
   __shared__ int s_len[kWideMaxSeqs];
   __shared__ int s_wpref[kSeqPlanMax + 1];
-  __shared__ int s_scan[NT / 64 + 1];
   __shared__ int s_redo;
   const int g = blockIdx.x;
   const int tid = threadIdx.x;
@@ -230,8 +229,8 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
 
   if (APPEND && p.len_out && g == 0)
     for (int b = tid; b < p.B; b += NT) p.len_out[b] = step_len_out(p.len_in, b, add, p.cap);
-  const Plan plan = plan_build<NT>(p.len_in, add, p.cap, p.B, 1, gridDim.x, s_pref, s_scan,
-                                   s_len, s_wpref, g, 1);
+  const Plan plan = plan_build(p.len_in, add, p.cap, p.B, 1, gridDim.x, s_pref, s_len, s_wpref, g,
+                               1);
   // sequences without tokens: the empty partial (0, -inf), or NaN for an
   // invalid length (spread over the workgroups, as in gqa_decode_kernel)
   for (int b = g; b < p.B; b += gridDim.x) {
@@ -257,8 +256,7 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
   const uint32_t sink_base = uniform((int)(uint32_t)(uintptr_t)&s_sink[0]);
 
   while (blk < blk_end) {
-    const int b = uniform((blk == blk_begin && plan.b0 >= 0) ? plan.b0
-                                                             : plan_seq(s_pref, p.B, blk));
+    const int b = uniform(blk == blk_begin ? plan.b0 : plan_seq(s_pref, p.B, blk));
     const int len = uniform(s_len[b]);
     const int len_old = len - add;
     const int row_start = uniform(s_pref[b]);

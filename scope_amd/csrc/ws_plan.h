@@ -25,8 +25,7 @@ struct Plan {
   int n;  // workgroups with work (min(grid, T)), at most 4096
   int q, r;  // T = q n + r
   bool seq;  // sequence-aligned ranges (plan_build with s_wpref)
-  // The calling split's range [begin, end) (when it passed its index g),
-  // and the sequence of block `begin` (-1: not known, use plan_seq).
+  // The calling split's range [begin, end) and the sequence of block `begin`.
   bool has_work;
   int begin, end, b0;
 };
@@ -35,7 +34,7 @@ struct Plan {
 // DPP sequence: every lane of the wave must be active.
 extern "C" __device__ int __ockl_wfscan_add_i32(int, bool);
 
-// Most sequences the sequence-aligned plan takes (one per lane).
+// Most sequences the sequence-aligned plan takes.
 constexpr int kSeqPlanMax = 64;
 // Blocks per split the sequence-aligned plan may add over ceil(T / n) and
 // still be chosen: a split whose range enters a second sequence restarts
@@ -91,88 +90,91 @@ __device__ __forceinline__ int plan_start(const Plan& p, int g) {
   return g * p.q + (int)((unsigned)(g * p.r) / (unsigned)p.n);
 }
 
+// The sequence-aligned plan's blocks per split: the smallest M in [base,
+// base + kAlignSlack], base = ceil(T / n), at which the sequences (lane b:
+// nb blocks) need at most n splits, or 0 if there is none.  The four
+// candidates are counted in one pass, summed over the wave as 16-bit halves
+// (each count is at most n + 64).  Every lane must call it.
+__device__ __forceinline__ int plan_align(int nb, const Plan& p) {
+  static_assert(kAlignSlack == 3, "four candidates, two per packed sum");
+  const int base = (p.T + p.n - 1) / p.n;
+  uint32_t c01 = 0, c23 = 0;
+  if (nb > 0) {
+    const uint32_t u = (uint32_t)nb;
+    c01 = (u + base - 1) / base | ((u + base) / (base + 1)) << 16;
+    c23 = (u + base + 1) / (base + 2) | ((u + base + 2) / (base + 3)) << 16;
+  }
+  c01 = __ockl_wfred_add_u32(c01);
+  c23 = __ockl_wfred_add_u32(c23);
+  const int cnt[4] = {(int)(c01 & 0xffffu), (int)(c01 >> 16), (int)(c23 & 0xffffu),
+                      (int)(c23 >> 16)};
+  int M = 0;
+#pragma unroll
+  for (int c = kAlignSlack; c >= 0; --c)
+    if (uniform(cnt[c]) <= p.n) M = base + c;
+  return M;
+}
+
 // Builds s_pref[0..B] (exclusive prefix of blocks per sequence, R rows each)
-// with the NT threads of the workgroup and returns the plan; with s_len, also
-// the lengths s_len[0..B) (plan_len), so callers need not read len_in again.
-// s_scan holds NT / 64 + 1 ints.  Every thread must call it.  With at most
-// 64 sequences every wave builds the whole plan by itself (lane b: sequence
-// b) and writes the same values, reading back only what it wrote: no barrier
-// between the kernel start and its first loads.  Otherwise the workgroup
-// builds it together, behind barriers.
+// and the lengths s_len[0..B) (plan_len), and returns the plan.  Every wave
+// of the workgroup calls it with all its lanes, builds the whole plan by
+// itself (lane b: sequence b; above 64 sequences, ceil(B / 64) consecutive
+// ones a lane) and writes the same values, reading back only what it wrote:
+// no barrier between the kernel start and its first loads.  (With more than
+// 64 sequences built together by the workgroup, behind three barriers and a
+// chain of one load per sequence of a lane, GQA B = 256 took 204.7 us a step,
+// against 187.5 with every wave on its own here and in the merge.)
 //
-// With s_wpref (kSeqPlanMax + 1 ints), one row per sequence (R == 1) and 2
-// to 64 sequences, the plan may instead be sequence-aligned: sequence b gets
-// n_b = ceil(nb(b) / M) splits, M the smallest block count per split with
-// sum_b n_b <= n, which take equal shares of its blocks, so no split spans
-// two sequences.  It is chosen when M <= ceil(T / n) + kAlignSlack (seq set,
-// s_wpref[b] = first split of sequence b, s_wpref[B] = splits used).  Every
-// kernel of a call (step and merge) passes the same arguments and so makes
-// the same choice.
+// With one row per sequence (R == 1) and 2 to 64 sequences, the plan may
+// instead be sequence-aligned: sequence b gets n_b = ceil(nb(b) / M) splits, M
+// the smallest block count per split with sum_b n_b <= n, which take equal
+// shares of its blocks, so no split spans two sequences.  It is chosen when
+// M <= ceil(T / n) + kAlignSlack (seq set, s_wpref[b] = first split of
+// sequence b, s_wpref[B] = splits used; kSeqPlanMax + 1 ints).  Every kernel
+// of a call (step and merge) passes the same arguments and so makes the same
+// choice.
 //
-// A split that passes its index g >= 0 gets its range in has_work / begin /
-// end (and, with at most 64 sequences, the sequence of its first block in
-// b0), computed from registers.
+// Split g (g >= 0) gets its range in has_work / begin / end and the sequence
+// of its first block in b0.
 //
 // ng > 1: B counts plan sequences v = b ng + group, whose lengths are
 // len_in[v / ng] (seq_of).
-template <int NT>
-__device__ Plan plan_build(const int32_t* len_in, int add, int cap, int B, int R,
-                           int grid, int* s_pref, int* s_scan, int* s_len = nullptr,
-                           int* s_wpref = nullptr, int g = -1, int ng = 1) {
-  constexpr int NW = NT / 64;
-  const int t = threadIdx.x;
-  const int lane = t & 63;
-  const int wave = t >> 6;
-  if (B >= 1 && B <= 64) {
+__device__ __forceinline__ Plan plan_build(const int32_t* len_in, int add, int cap, int B, int R,
+                                           int grid, int* s_pref, int* s_len, int* s_wpref,
+                                           int g, int ng) {
+  const int lane = threadIdx.x & 63;
+  if (__builtin_expect(B >= 1 && B <= 64, 1)) {
     const int l = lane < B ? plan_len(len_in, seq_of(lane, ng), add, cap) : 0;
     const int nb = R * ((l + 31) >> 5);
     const int incl = __ockl_wfscan_add_i32(nb, true);
     if (lane < B) {
       s_pref[lane] = incl - nb;
-      if (s_len) s_len[lane] = l;
+      s_len[lane] = l;
     }
     const int T = __builtin_amdgcn_readlane(incl, B - 1);
     if (lane == 0) s_pref[B] = T;
     Plan p = plan_of(T, grid);
-    if (s_wpref && R == 1 && B >= 2 && p.n > 0) {
-      // splits needed with M = base + c blocks per split, c = 0..3, summed
-      // over the wave as four 16-bit counts (each at most n + 64)
-      const int base = (T + p.n - 1) / p.n;
-      uint32_t c01 = 0, c23 = 0;
-      if (nb > 0) {
-        const uint32_t u = (uint32_t)nb;
-        c01 = (u + base - 1) / base | ((u + base) / (base + 1)) << 16;
-        c23 = (u + base + 1) / (base + 2) | ((u + base + 2) / (base + 3)) << 16;
+    const int M = R == 1 && B >= 2 && p.n > 0 ? plan_align(nb, p) : 0;
+    if (M > 0) {
+      const int ns = nb > 0 ? (nb + M - 1) / M : 0;
+      const int w = __ockl_wfscan_add_i32(ns, true);
+      const int used = __builtin_amdgcn_readlane(w, B - 1);
+      if (lane < B) s_wpref[lane] = w - ns;
+      if (lane == 0) s_wpref[B] = used;
+      p.seq = true;
+      if (g >= 0 && g < used) {
+        // split g: sequence b (the first with w > g), its j-th of ns splits
+        const int b = __builtin_ctzll(__builtin_amdgcn_ballot_w64(lane < B && w > g));
+        const int j = g - (__builtin_amdgcn_readlane(w, b) - __builtin_amdgcn_readlane(ns, b));
+        const int nsb = __builtin_amdgcn_readlane(ns, b);
+        const int first = __builtin_amdgcn_readlane(incl, b) - __builtin_amdgcn_readlane(nb, b);
+        const int nbb = __builtin_amdgcn_readlane(nb, b);
+        p.has_work = true;
+        p.begin = first + j * nbb / nsb;
+        p.end = first + (j + 1) * nbb / nsb;
+        p.b0 = b;
       }
-      c01 = __ockl_wfred_add_u32(c01);
-      c23 = __ockl_wfred_add_u32(c23);
-      const int cnt[4] = {(int)(c01 & 0xffffu), (int)(c01 >> 16), (int)(c23 & 0xffffu),
-                          (int)(c23 >> 16)};
-      int M = 0;
-#pragma unroll
-      for (int c = kAlignSlack; c >= 0; --c)
-        if (uniform(cnt[c]) <= p.n) M = base + c;
-      if (M > 0) {
-        const int ns = nb > 0 ? (nb + M - 1) / M : 0;
-        const int w = __ockl_wfscan_add_i32(ns, true);
-        const int used = __builtin_amdgcn_readlane(w, B - 1);
-        if (lane < B) s_wpref[lane] = w - ns;
-        if (lane == 0) s_wpref[B] = used;
-        p.seq = true;
-        if (g >= 0 && g < used) {
-          // split g: sequence b (the first with w > g), its j-th of ns splits
-          const int b = __builtin_ctzll(__builtin_amdgcn_ballot_w64(lane < B && w > g));
-          const int j = g - (__builtin_amdgcn_readlane(w, b) - __builtin_amdgcn_readlane(ns, b));
-          const int nsb = __builtin_amdgcn_readlane(ns, b);
-          const int first = __builtin_amdgcn_readlane(incl, b) - __builtin_amdgcn_readlane(nb, b);
-          const int nbb = __builtin_amdgcn_readlane(nb, b);
-          p.has_work = true;
-          p.begin = first + j * nbb / nsb;
-          p.end = first + (j + 1) * nbb / nsb;
-          p.b0 = b;
-        }
-        return p;
-      }
+      return p;
     }
     if (g >= 0 && g < p.n) {
       p.has_work = true;
@@ -182,50 +184,44 @@ __device__ Plan plan_build(const int32_t* len_in, int add, int cap, int B, int R
     }
     return p;
   }
-  const int chunk = (B + NT - 1) / NT;
-  const int b0 = min(B, t * chunk);
-  const int b1 = min(B, b0 + chunk);
-  int local = 0;
-  for (int b = b0; b < b1; ++b) {
-    const int l = plan_len(len_in, seq_of(b, ng), add, cap);
-    if (s_len) s_len[b] = l;
-    local += R * ((l + 31) >> 5);
-  }
-  // inclusive scan of `local` across the wave
-  int incl = local;
+  // lane: sequences c * lane .. c * lane + c - 1, four loads at a time
+  const int c = (B + 63) >> 6;
+  const int v0 = c * lane;
+  int sum = 0;
+  for (int k0 = 0; k0 < c; k0 += 4) {
+    int l[4];
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int v = __shfl_up(incl, o);
-    if (lane >= o) incl += v;
-  }
-  if (lane == 63) s_scan[wave] = incl;
-  __syncthreads();
-  if (t == 0) {
-    int run = 0;
-    for (int w = 0; w < NW; ++w) {
-      const int v = s_scan[w];
-      s_scan[w] = run;
-      run += v;
+    for (int k = 0; k < 4; ++k)
+      l[k] = plan_len(len_in, seq_of(min(v0 + k0 + k, B - 1), ng), add, cap);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (k0 + k >= c || v0 + k0 + k >= B) continue;
+      s_len[v0 + k0 + k] = l[k];
+      sum += R * ((l[k] + 31) >> 5);
     }
-    s_scan[NW] = run;
   }
-  __syncthreads();
-  int run = s_scan[wave] + incl - local;
-  for (int b = b0; b < b1; ++b) {
-    s_pref[b] = run;
-    run += R * (((s_len ? s_len[b] : plan_len(len_in, seq_of(b, ng), add, cap)) + 31) >> 5);
+  const int incl = __ockl_wfscan_add_i32(sum, true);
+  // (only final values go to LDS: the workgroup's waves all write them)
+  int run = incl - sum;
+  for (int k = 0; k < min(c, B - v0); ++k) {
+    s_pref[v0 + k] = run;
+    run += R * ((s_len[v0 + k] + 31) >> 5);
   }
-  if (t == 0) s_pref[B] = s_scan[NW];
-  __syncthreads();
-  Plan p = plan_of(uniform(s_scan[NW]), grid);
+  const int T = __builtin_amdgcn_readlane(incl, 63);
+  if (lane == 0) s_pref[B] = T;
+  Plan p = plan_of(T, grid);
   if (g >= 0 && g < p.n) {
     p.has_work = true;
     p.begin = plan_start(p, g);
     p.end = plan_start(p, g + 1);
+    // the lane with the first sequence that ends past block `begin`, then the
+    // sequence among its c <= 32
+    const int vb = c * __builtin_ctzll(__builtin_amdgcn_ballot_w64(incl > p.begin));
+    const bool past = lane < c && vb + lane < B && s_pref[min(vb + lane + 1, B)] <= p.begin;
+    p.b0 = vb + __builtin_popcountll(__builtin_amdgcn_ballot_w64(past));
   }
   return p;
 }
-
 
 // Workgroup whose range holds block blk: ceil((blk + 1) n / T) - 1.  The
 // double quotient is exact enough: the operands are integers below 2^53, and
@@ -235,18 +231,71 @@ __device__ __forceinline__ int plan_owner(const Plan& p, int blk) {
   return (int)ceil((double)(blk + 1) * (double)p.n / (double)p.T) - 1;
 }
 
-// Splits holding row `row` (sequence b under a sequence-aligned plan, whose
-// rows are sequences), blocks [row_start, row_start + nbb), nbb >= 1: the
-// first split and how many.
-__device__ __forceinline__ void plan_row_splits(const Plan& p, int b, int row_start, int nbb,
-                                                const int* s_wpref, int& w_first, int& nseg) {
-  if (p.seq) {
-    w_first = s_wpref[b];
-    nseg = s_wpref[b + 1] - s_wpref[b];
-  } else {
-    w_first = plan_owner(p, row_start);
-    nseg = plan_owner(p, row_start + nbb - 1) - w_first + 1;
+// What a merge needs of the plan: the pieces of one row.
+struct RowSplits {
+  int nbb;      // the row's blocks (0: no pieces, its partial is in out / lse)
+  int w_first;  // its first split
+  int nseg;     // and how many splits hold it
+};
+
+// The pieces of row r of plan sequence v under plan_build's plan, from wave
+// sums over the lengths: no prefix in LDS and no barrier, so a merge's start
+// costs one coalesced load of the lengths, whatever the batch (a merge
+// workgroup per output row that rebuilt the whole prefix made the merge of
+// 256 sequences x 32 heads 24 us, and of 96 sequences x 8 head groups 116).
+// Every lane of the wave must be active; v and r are wave-uniform.
+template <int K>
+__device__ __forceinline__ RowSplits plan_row_k(const int32_t* len_in, int add, int cap, int B,
+                                                int R, int grid, int v, int r, int ng) {
+  const int lane = threadIdx.x & 63;
+  int nb[K];
+  uint32_t sum = 0, before = 0;
+  RowSplits rs{0, 0, 0};
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int u = lane + 64 * k;
+    int l = plan_len(len_in, seq_of(min(u, B - 1), ng), add, cap);
+    if (u >= B) l = 0;
+    nb[k] = (l + 31) >> 5;
+    sum += nb[k];
+    before += u < v ? nb[k] : 0;
+    if (k == (v >> 6)) rs.nbb = __builtin_amdgcn_readlane(nb[k], v & 63);
   }
+  if (rs.nbb == 0) return rs;
+  const Plan p = plan_of(R * uniform((int)__ockl_wfred_add_u32(sum)), grid);
+  const int M = K == 1 && R == 1 && B >= 2 ? plan_align(nb[0], p) : 0;
+  if (M > 0) {
+    rs.w_first =
+        uniform((int)__ockl_wfred_add_u32(lane < v ? ((uint32_t)nb[0] + M - 1) / M : 0u));
+    rs.nseg = (rs.nbb + M - 1) / M;
+  } else {
+    const int start = R * uniform((int)__ockl_wfred_add_u32(before)) + r * rs.nbb;
+    rs.w_first = plan_owner(p, start);
+    rs.nseg = plan_owner(p, start + rs.nbb - 1) - rs.w_first + 1;
+  }
+  return rs;
+}
+__device__ __forceinline__ RowSplits plan_row(const int32_t* len_in, int add, int cap, int B,
+                                              int R, int grid, int v, int r, int ng) {
+  if (B <= 64) return plan_row_k<1>(len_in, add, cap, B, R, grid, v, r, ng);
+  if (B <= 256) return plan_row_k<4>(len_in, add, cap, B, R, grid, v, r, ng);
+  const int lane = threadIdx.x & 63;
+  uint32_t sum = 0, before = 0;
+#pragma unroll 4
+  for (int u = lane; u < B; u += 64) {
+    const int nb = (plan_len(len_in, seq_of(u, ng), add, cap) + 31) >> 5;
+    sum += nb;
+    before += u < v ? nb : 0;
+  }
+  RowSplits rs{(plan_len(len_in, seq_of(v, ng), add, cap) + 31) >> 5, 0, 0};
+  const uint32_t tot = __ockl_wfred_add_u32(sum);
+  const uint32_t bef = __ockl_wfred_add_u32(before);
+  if (rs.nbb == 0) return rs;
+  const Plan p = plan_of(R * uniform((int)tot), grid);
+  const int start = R * uniform((int)bef) + r * rs.nbb;
+  rs.w_first = plan_owner(p, start);
+  rs.nseg = plan_owner(p, start + rs.nbb - 1) - rs.w_first + 1;
+  return rs;
 }
 
 // Sequence holding block blk: the last b with s_pref[b] <= blk (B >= 1).
