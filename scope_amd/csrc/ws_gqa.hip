@@ -162,7 +162,6 @@ gqa_decode_kernel(
   constexpr int add = APPEND ? 1 : 0;
   __shared__ int s_pref[kMaxSeqs + 1];
   __shared__ int s_len[kMaxSeqs];
-  __shared__ int s_wpref[kSeqPlanMax + 1];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -175,8 +174,8 @@ gqa_decode_kernel(
   if (APPEND && p.len_out && blockIdx.x == 0)
     for (int b = tid; b < p.B; b += NT) p.len_out[b] = step_len_out(p.len_in, b, add, p.cap);
   const Plan plan =
-      plan_build(p.len_in, add, p.cap, p.B, p.Hkv, p.n_splits, s_pref, s_len, s_wpref,
-                 uniform(blockIdx.x * W + (tid >> 6)), 1);
+      plan_build(p.len_in, add, p.cap, p.B, p.Hkv, p.n_splits, s_pref, s_len,
+                 uniform(blockIdx.x * W + (tid >> 6)), 1, kAlignStep);
   // Sequences without tokens: the empty partial (0, -inf), or NaN for an
   // invalid length.  Workgroup g looks at sequences g, g + grid, ...: one
   // workgroup looking at all of them is a chain of an LDS read per sequence

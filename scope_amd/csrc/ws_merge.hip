@@ -101,6 +101,7 @@ struct MergeSplitParams {
   // B: plan sequences; ng > 1 for absorbed MLA with H = 16 ng heads, whose
   // plan sequences are (sequence, 16-head group) pairs (ws_plan.h seq_of).
   int B, ng, R, heads, Dv, cap, grid;
+  int step;  // the plan's alignment step
   int add;  // lengths are gpu_len[b] + add (1 when gpu_len is a fused step's len_in)
   const float* out_g;
   const float* lse_g;
@@ -142,7 +143,7 @@ __global__ __launch_bounds__(64) void merge_split_kernel(const MergeSplitParams 
   if (FMT >= 0)
     load_b<(FMT >= 0 ? FMT : 0)>(p.b_out, p.b_aux0, p.b_aux1, qrow, p.Dv, col_ok ? c : 0, lb,
                                  ob);
-  const RowSplits rs = plan_row(p.gpu_len, p.add, p.cap, p.B, p.R, p.grid, b, r, p.ng);
+  const RowSplits rs = plan_row(p.gpu_len, p.add, p.cap, p.B, p.R, p.grid, b, r, p.ng, p.step);
   // One piece: the step's final partial (out_g, fp32); several: their bf16
   // workspace slots, piece s at pieces + s * sstride.
   int n = 1;
@@ -258,7 +259,7 @@ __global__ __launch_bounds__(kUvThreads) void merge_split_uv_kernel(
   float4 ob = make_float4(0.f, 0.f, 0.f, 0.f);
   if (FMT >= 0 && merging)
     load_b<(FMT >= 0 ? FMT : 0)>(p.b_out, p.b_aux0, p.b_aux1, qrow, p.Dv, c, lb, ob);
-  const RowSplits rs = plan_row(p.gpu_len, p.add, p.cap, p.B, 1, p.grid, pv_seq, 0, p.ng);
+  const RowSplits rs = plan_row(p.gpu_len, p.add, p.cap, p.B, 1, p.grid, pv_seq, 0, p.ng, p.step);
   int n = 1;
   const float* src = p.out_g + (size_t)qrow * p.Dv;
   const uint16_t* pieces = nullptr;
@@ -380,6 +381,7 @@ int merge_split_pieces(const int32_t* len, int len_add, int B, int R, int heads,
   prm.gpu_len = len;
   prm.B = B;
   prm.ng = 1;
+  prm.step = kAlignStep;
   prm.R = R;
   prm.heads = heads;
   prm.Dv = Dv;
@@ -427,7 +429,8 @@ extern "C" int ws_merge_split(const int32_t* gpu_len, int B, int rows_per_seq, i
   // an absorbed-MLA step with H = 16 ng heads planned (sequence, head group)
   // pairs, unless its layout is wide (ws_reduce.h mla_layout)
   const bool mla = Dv == 512 && rows_per_seq == 1 && heads > 16 && heads % 16 == 0;
-  const int ng = mla ? mla_layout(B, heads).ng : 1;
+  const MlaLayout lay = mla_layout(B, heads);
+  const int ng = mla ? lay.ng : 1;
   if (B < 0 || (long long)B * ng > kMaxSeqs || rows_per_seq <= 0 || heads <= 0 ||
       (heads > 16 && !mla) || Dv <= 0 || Dv % 4 || Dv > 512 || page_capacity <= 0 ||
       n_workgroups <= 0)
@@ -460,6 +463,7 @@ extern "C" int ws_merge_split(const int32_t* gpu_len, int B, int rows_per_seq, i
   prm.R = rows_per_seq;
   prm.heads = heads;
   prm.Dv = Dv;
+  prm.step = mla ? lay.step : kAlignStep;
   prm.cap = page_capacity;
   prm.grid = n_workgroups;
   prm.add = 0;
@@ -585,6 +589,7 @@ extern "C" int ws_mla_merge_split_uv(const int32_t* gpu_len, int B, int heads,
   prm.R = 1;
   prm.heads = heads;
   prm.Dv = Dv;
+  prm.step = lay.step;
   prm.cap = page_capacity;
   prm.grid = n_workgroups;
   prm.add = 0;

@@ -52,9 +52,10 @@ struct MlaParams {
   float* part_lse;     // [slot][16]
   // B: plan sequences v = b * ng + g, one per (sequence b, 16-head group g);
   // rows of q / out are v * 16 + h, i.e. b * H + 16 g + h with H = 16 ng.
-  // The wide kernel plans sequences (ng = 1) with 128-head rows.
+  // The wide kernel plans sequences (ng = 1) with rows of all H heads.
   int B, ng, page_size, max_pages, num_pages, cap;
-  int hp;  // heads of a piece (and of a plan sequence's rows): 16, or 128 (wide)
+  int hp;  // heads of a piece (and of a plan sequence's rows): 16, or all H (wide)
+  int step;  // the plan's alignment step
   float scale_log2;
 };
 
@@ -103,7 +104,6 @@ __global__ __launch_bounds__(256) void mla_decode_kernel(const MlaParams p) {
   __shared__ f32x4 sbuf[2][2][2][64];      // [block parity][latent half][token tile][lane]
   __shared__ int s_pref[kMaxSeqs + 1];
   __shared__ int s_len[kMaxSeqs];
-  __shared__ int s_wpref[kSeqPlanMax + 1];
   const int g = blockIdx.x;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -122,8 +122,8 @@ __global__ __launch_bounds__(256) void mla_decode_kernel(const MlaParams p) {
   if (APPEND && p.len_out && g == 0)
     for (int b = tid; b < p.B / p.ng; b += NT)
       p.len_out[b] = step_len_out(p.len_in, b, add, p.cap);
-  const Plan plan = plan_build(p.len_in, add, p.cap, p.B, 1, gridDim.x, s_pref, s_len, s_wpref, g,
-                               p.ng);
+  const Plan plan = plan_build(p.len_in, add, p.cap, p.B, 1, gridDim.x, s_pref, s_len, g, p.ng,
+                               kAlignStep);
   // sequences without tokens: the empty partial (0, -inf), or NaN for an
   // invalid length (spread over the workgroups, as in gqa_decode_kernel)
   for (int b = g; b < p.B; b += gridDim.x) {
@@ -423,7 +423,7 @@ __global__ __launch_bounds__(64) void mla_reduce_kernel(const MlaParams p, int g
   const int b = hrow / p.hp;
   const int h = hrow - b * p.hp;
   const int add = p.c_new ? 1 : 0;
-  const RowSplits rs = plan_row(p.len_in, add, p.cap, p.B, 1, grid, b, 0, p.ng);
+  const RowSplits rs = plan_row(p.len_in, add, p.cap, p.B, 1, grid, b, 0, p.ng, p.step);
   const int n = rs.nseg;
   if (n <= 1) return;
   const size_t slot0 = (size_t)(rs.w_first + b) * p.hp + h;  // partial row of split 0
@@ -461,10 +461,12 @@ static bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 // Workgroups of an MLA call: n_workgroups when given, else one per CU (the
 // kernel's occupancy), at most what the blocks of the longest possible batch
-// can feed with 4 blocks each, and no more than the reduction's weights hold.
+// can feed with 4 blocks each, or one per plan sequence (B) where that is more
+// (sequences of one to three blocks), and no more than the reduction's weights
+// hold.
 int mla_workgroups(int n_workgroups, int B, int max_len) {
   if (n_workgroups > 0) return n_workgroups;
-  const long long max_blocks = (long long)B * ((max_len + 31) / 32);
+  const long long max_blocks = (long long)B * std::max((max_len + 31) / 32, 4);
   const int n = choose_workgroups(0, 1, max_blocks, 4);
   return std::min(n, kReduceMaxWeights);
 }
@@ -484,8 +486,8 @@ static int mla_launch(const uint16_t* q_nope, const uint16_t* q_pe,
     return set_error(WS_EINVAL,
                      "%s: B=%d H=%d unsupported (H a multiple of 16, B * H / 16 <= %d)", name, B,
                      H, kMaxSeqs);
-  // 128 heads over at most 64 sequences: the wide kernel, one plan sequence
-  // per sequence and 128-head pieces (ws_reduce.h mla_layout)
+  // the wide kernel: one plan sequence per sequence and pieces of all heads
+  // (ws_reduce.h mla_layout)
   const MlaLayout lay = mla_layout(B, H);
   const int ng = lay.ng;
   if (page_size <= 0 || max_pages <= 0 || num_pages <= 0 || max_len < 0 ||
@@ -541,6 +543,7 @@ static int mla_launch(const uint16_t* q_nope, const uint16_t* q_pe,
   prm.B = Bv;
   prm.ng = ng;
   prm.hp = hp;
+  prm.step = lay.step;
   prm.page_size = page_size;
   prm.max_pages = max_pages;
   prm.num_pages = num_pages;
@@ -548,10 +551,10 @@ static int mla_launch(const uint16_t* q_nope, const uint16_t* q_pe,
   prm.scale_log2 = scale * kLog2e;
   hipStream_t s = (hipStream_t)stream;
   if (lay.wide) {
-    if (c_new)
-      hipLaunchKernelGGL(mla_wide_kernel<true>, dim3(n), dim3(256), 0, s, prm);
-    else
-      hipLaunchKernelGGL(mla_wide_kernel<false>, dim3(n), dim3(256), 0, s, prm);
+    const bool full = H == kWideHeads;
+    const auto kernel = c_new ? (full ? mla_wide_kernel<true, true> : mla_wide_kernel<true, false>)
+                              : (full ? mla_wide_kernel<false, true> : mla_wide_kernel<false, false>);
+    hipLaunchKernelGGL(kernel, dim3(n), dim3(256), 0, s, prm);
   } else if (c_new) {
     hipLaunchKernelGGL(mla_decode_kernel<true>, dim3(n), dim3(256), 0, s, prm);
   } else {

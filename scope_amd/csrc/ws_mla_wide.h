@@ -1,7 +1,7 @@
-// Split-KV absorbed-MLA decode attention with 128 query heads (DeepSeek-V2)
-// over the HBM partition (gfx950), optionally fused with the append of the
-// decode step's new latent.  Included by ws_mla.hip, which dispatches calls
-// whose layout is wide (ws_reduce.h mla_layout) here.
+// Split-KV absorbed-MLA decode attention with up to 128 query heads
+// (DeepSeek-V2) over the HBM partition (gfx950), optionally fused with the
+// append of the decode step's new latent.  Included by ws_mla.hip, which
+// dispatches calls whose layout is wide (ws_reduce.h mla_layout) here.
 //
 // The 16-head kernel would stream the shared latent once per 16-head group.
 // Here every 32-token latent block is read from HBM once per workgroup and
@@ -56,10 +56,14 @@
 // usual relative precision (both reach 2^127).  A segment whose scores climb
 // further above m_ref runs again with the true maximum as the reference.
 //
-// Plan (ws_plan.h) over sequences (at most 64); a sequence held by one
-// workgroup is written final (fp32 out / lse), otherwise each workgroup
-// leaves a bf16 piece of all 128 heads in slot workgroup + sequence, which
-// mla_reduce_kernel or the merges combine.
+// Plan (ws_plan.h) over sequences; a sequence held by one workgroup is written
+// final (fp32 out / lse), otherwise each workgroup leaves a bf16 piece of all
+// its heads in slot workgroup + sequence, which mla_reduce_kernel or the merges
+// combine.  A workgroup that enters a second sequence pays a start and an end
+// again (about 14 us: ten blocks' time), so the plan prefers ranges of one
+// sequence (kAlignStepWide).  128 heads, B = 96 of 256 to 4096 tokens, step and
+// merge: 380 us as eight 16-head groups a sequence, 103 here; B = 40 of 500 to
+// 4000 tokens 75 -> 59 us by the alignment.
 #pragma once
 
 namespace ws {
@@ -167,13 +171,14 @@ __device__ __forceinline__ void wide_lds_wait() {
   asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
 }
 
-// Stores 32 staged 1 KB rows (row h at src + 260 h dwords, lane part at
-// src) to dst + h * row_bytes + col_byte, eight rows' LDS reads in flight
-// before their stores.
+// Stores `rows` (0, 16 or 32) staged 1 KB rows (row h at src + 260 h dwords,
+// lane part at src) to dst + h * row_bytes + col_byte, eight rows' LDS reads in
+// flight before their stores.
 __device__ __forceinline__ void wide_store_rows(char* dst, int row_bytes, const uint32_t* src,
-                                                int col_byte) {
+                                                int col_byte, int rows) {
 #pragma unroll
   for (int h0 = 0; h0 < 32; h0 += 8) {
+    if (h0 >= rows) break;
     u32x4 v[8];
 #pragma unroll
     for (int h = 0; h < 8; ++h) v[h] = *(const u32x4*)(src + (h0 + h) * 260);
@@ -183,16 +188,17 @@ __device__ __forceinline__ void wide_store_rows(char* dst, int row_bytes, const 
   }
 }
 
-template <bool APPEND>
+// FULL: 128 heads (known at compile time: B = 1 with 16k tokens 29.3 us a step
+// with its merge, 30.6 with the head count read at run time).
+template <bool APPEND, bool FULL>
 __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
   constexpr int NT = 256;
-  constexpr int H = kWideHeads;
+  const int H = FULL ? kWideHeads : p.hp;  // a multiple of 16 from kWideMinHeads to kWideHeads
   constexpr int add = APPEND ? 1 : 0;
   __shared__ u32x4 s_tile[kWideTiles][kWideTileAlloc];
   __shared__ u32x4 s_sink[64];
   __shared__ int s_pref[kWideMaxSeqs + 1];
   __shared__ int s_len[kWideMaxSeqs];
-  __shared__ int s_wpref[kSeqPlanMax + 1];
   __shared__ int s_redo;
   const int g = blockIdx.x;
   const int tid = threadIdx.x;
@@ -201,6 +207,10 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
   const int n32 = lane & 31;  // head (QK B, PV B, output) or row (A operands)
   const int j2 = lane >> 5;   // k-slot half
   const int head = 32 * wave + n32;
+  // Fewer than 128 heads: a wave whose last 16 columns are past the heads
+  // repeats the last one there (MFMA columns are independent) and does not
+  // store them; a wave without heads only loads its part of the blocks.
+  const int rows = FULL ? 32 : min(max(H - 32 * wave, 0), 32);  // this wave's heads
   // Byte offsets, within a block of 32 consecutive token rows in HBM, of the
   // chunks this lane loads with its kWideDmaPerWave instructions (tile chunk
   // c of row r = wide_row_of(c) is chunk c - wide_row_off(r) of the row; pad
@@ -229,8 +239,8 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
 
   if (APPEND && p.len_out && g == 0)
     for (int b = tid; b < p.B; b += NT) p.len_out[b] = step_len_out(p.len_in, b, add, p.cap);
-  const Plan plan = plan_build(p.len_in, add, p.cap, p.B, 1, gridDim.x, s_pref, s_len, s_wpref, g,
-                               1);
+  const Plan plan = plan_build(p.len_in, add, p.cap, p.B, 1, gridDim.x, s_pref, s_len, g, 1,
+                               kAlignStepWide);
   // sequences without tokens: the empty partial (0, -inf), or NaN for an
   // invalid length (spread over the workgroups, as in gqa_decode_kernel)
   for (int b = g; b < p.B; b += gridDim.x) {
@@ -274,27 +284,30 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
     int pid_base = 0;
     int m_tok = 0;
     int seg_bad = 0;
-    auto fetch_pids = [&]() __attribute__((always_inline)) {
-      const int t0 = t_begin + 32 * min(pid_base + lane, nblk - 1);
+    auto first_tok = [&]() __attribute__((always_inline)) {
+      return t_begin + 32 * min(pid_base + lane, nblk - 1);
+    };
+    auto set_pids = [&](int raw) __attribute__((always_inline)) {
+      const int t0 = first_tok();
       const int page = t0 / p.page_size;
-      const int raw = pt[page];
       const int pid = clamp_page(raw, p.num_pages);
       m_tok = (pid * p.page_size + (t0 - page * p.page_size)) |
               (raw == pid ? 0 : (int)0x80000000u);
     };
-    fetch_pids();
+    auto fetch_pids = [&]() __attribute__((always_inline)) {
+      set_pids(pt[first_tok() / p.page_size]);
+    };
+    // The first ones are requested here and used after the queries are in, so
+    // that their round trip is not added to the queries'.
+    int raw_pid = pt[first_tok() / p.page_size];
     // The appended token is its sequence's last, so one segment holds it: that
     // segment's workgroup writes its row (c_new, pe_new) into the token's page
     // slot first, and every block then loads from the pool alike.
     const bool owner = APPEND && len_old >= t_begin && len_old < t_end;
     u32x4 new_chunk = {0u, 0u, 0u, 0u};
-    int new_dst = -1;  // the row's pool token index, -1: not written here
+    int new_pid = -1;  // the row's page, -1: not written here
     if (owner && tid < kWideRowData) {
-      const int page = len_old / p.page_size;
-      const int raw = pt[page];
-      new_dst = clamp_page(raw, p.num_pages) == raw
-                    ? raw * p.page_size + (len_old - page * p.page_size)
-                    : -1;
+      new_pid = pt[len_old / p.page_size];
       new_chunk = tid < kMlaC / 8
                       ? ((const u32x4*)(p.c_new + (size_t)b * p.c_stride))[tid]
                       : ((const u32x4*)(p.pe_new + (size_t)b * p.pe_stride))[tid - kMlaC / 8];
@@ -307,16 +320,25 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
     // the q_pe chunks are loaded straight into registers.
     u32x4 qb[36];
     {
-      const size_t qrow0 = (size_t)b * H + 32 * wave;
+      const uint16_t* qrow0 = p.q_nope + ((size_t)b * H + 32 * wave) * kMlaC;
       const uint32_t qst = tile_base0 + (uint32_t)(32 * wave * 65 * 16);
+      if (rows == 32) {
 #pragma unroll 8
-      for (int h = 0; h < 32; ++h)
-        wide_dma16_s(16 * lane, p.q_nope + (qrow0 + h) * kMlaC, qst + (uint32_t)(h * 65 * 16));
+        for (int h = 0; h < 32; ++h)
+          wide_dma16_s(16 * lane, qrow0 + h * kMlaC, qst + (uint32_t)(h * 65 * 16));
+      } else if (rows > 0) {
+        for (int h = 0; h < 32; ++h)
+          wide_dma16_s(16 * lane, qrow0 + min(h, rows - 1) * kMlaC, qst + (uint32_t)(h * 65 * 16));
+      }
 #pragma unroll
       for (int u = 32; u < 36; ++u)
-        qb[u] = ((const u32x4*)(p.q_pe + (qrow0 + n32) * 64))[2 * (u - 32) + j2];
-      asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-      if (new_dst >= 0) ((u32x4*)(p.latent_w + (size_t)new_dst * kMlaL))[tid] = new_chunk;
+        qb[u] = ((const u32x4*)(p.q_pe + ((size_t)b * H + min(head, H - 1)) * 64))[2 * (u - 32) + j2];
+      asm volatile("s_waitcnt vmcnt(0)" : "+v"(raw_pid), "+v"(new_pid) : : "memory");
+      set_pids(raw_pid);
+      if (new_pid >= 0 && new_pid < p.num_pages)
+        ((u32x4*)(p.latent_w +
+                  ((size_t)new_pid * p.page_size + len_old % p.page_size) * kMlaL))[tid] =
+            new_chunk;
       const u32x4* qs = &s_tile[0][0] + (32 * wave + n32) * 65 + j2;
 #pragma unroll
       for (int u = 0; u < 32; ++u) qb[u] = qs[2 * u];
@@ -401,7 +423,8 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
     f32x16 acc[16];
     float m_run = neg_inf();  // reference max (m_ref) of the lane's head
     float m_max = neg_inf();  // the lane's largest score of the segment so far
-    float l_run = 0.f;
+    float l_run = 0.f;  // the lane's sum of probabilities as rounded
+    float s_run = 0.f;  // and in fp32
 
     // Pieces of the ring (block k in tile k % 4):
     //   QK(k)    36 MFMAs into sc; A = row n32 of the tile, k-step u = chunk
@@ -486,11 +509,14 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
       }
     };
     // soft_p: one dword of a k-step's P^T (two exp2), its two probabilities
-    // added to the row sum as rounded (the PV MFMAs see the same values)
+    // added to the row sums: as rounded (the values the PV MFMAs see), which
+    // normalises the outputs, and in fp32 for the lse
     auto soft_p = [&](const float (&xs)[8], u32x4& pbs, int dd) __attribute__((always_inline)) {
       typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-      const uint32_t pk = pack_bf16x2(__builtin_amdgcn_exp2f(xs[2 * dd]),
-                                      __builtin_amdgcn_exp2f(xs[2 * dd + 1]));
+      const float p0 = __builtin_amdgcn_exp2f(xs[2 * dd]);
+      const float p1 = __builtin_amdgcn_exp2f(xs[2 * dd + 1]);
+      const uint32_t pk = pack_bf16x2(p0, p1);
+      s_run += p0 + p1;
       pbs[dd] = pk;
       l_run = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, pk),
                                               __builtin_bit_cast(bf16x2_t, 0x3f803f80u), l_run,
@@ -568,6 +594,7 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[e][i] = 0.f;
       l_run = 0.f;
+      s_run = 0.f;
       if (pid_base != 0) {
         pid_base = 0;
         fetch_pids();
@@ -575,23 +602,32 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
       issue(0, 0);
       issue(1, 1);
       issue(2, 2);
-      float xa[8], xh[8];
-      {  // QK and soft_x of block 0
-        wide_wait_barrier<2 * kWideDmaPerWave>();
-        f32x16 sc;
-        u32x4 kr[5];
+      if (rows > 0) {
+        float xa[8], xh[8];
+        {  // QK and soft_x of block 0
+          wide_wait_barrier<2 * kWideDmaPerWave>();
+          f32x16 sc;
+          u32x4 kr[5];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) kr[u] = qk_read(0, u);
+          for (int u = 0; u < 4; ++u) kr[u] = qk_read(0, u);
 #pragma unroll
-        for (int u = 0; u < 36; ++u) {
-          if (u + 4 < 36) kr[(u + 4) % 5] = qk_read(0, u + 4);
-          qk_mfma(sc, kr[u % 5], u);
+          for (int u = 0; u < 36; ++u) {
+            if (u + 4 < 36) kr[(u + 4) % 5] = qk_read(0, u + 4);
+            qk_mfma(sc, kr[u % 5], u);
+          }
+          soft_x(0, sc, xa, xh, true);
         }
-        soft_x(0, sc, xa, xh, true);
-      }
 #pragma clang loop unroll(disable)
-      for (int k = 0; k + 1 < nblk; ++k) step(k, xa, xh);
-      step_last(nblk - 1, xa, xh);
+        for (int k = 0; k + 1 < nblk; ++k) step(k, xa, xh);
+        step_last(nblk - 1, xa, xh);
+      } else {  // the ring's waits, barriers and loads alone
+        wide_wait_barrier<2 * kWideDmaPerWave>();
+#pragma clang loop unroll(disable)
+        for (int k = 0; k + 1 < nblk; ++k) {
+          wide_wait_barrier<kWideDmaPerWave>();
+          issue(k + 3, (k + 3) & (kWideTiles - 1));
+        }
+      }
       {  // the head's largest score (both lanes of the head)
         float lo, hi;
         pair_xor32(m_max, lo, hi);
@@ -614,11 +650,13 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
     float lo, hi;
     pair_xor32(l_run, lo, hi);
     const float l_tot = lo + hi;
+    pair_xor32(s_run, lo, hi);
+    const float s_tot = lo + hi;
     const bool bad = seg_bad < 0;  // a bad page id was read (clamped): the piece is NaN
     const float inv_l = bad ? qnan() : 1.f / l_tot;
-    const float lse_v = bad ? qnan() : (m_run + __log2f(l_tot)) * kLn2;
+    const float lse_v = bad ? qnan() : (m_run + __log2f(s_tot)) * kLn2;
     const bool whole = row_start >= blk_begin && row_end <= blk_end;  // final, fp32
-    if (j2 == 0) {
+    if (j2 == 0 && n32 < rows) {
       if (whole)
         p.lse[(size_t)b * H + head] = lse_v;
       else
@@ -631,7 +669,8 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
     // two lanes per bank pair) and stores them itself.  Accumulator ct value
     // i is column 32 ct + 8 (i / 4) + 4 j2 + i % 4.
     uint32_t* stage = (uint32_t*)&s_tile[0][0] + (size_t)(32 * wave) * 260;
-    if (!whole) {  // bf16 piece: all 512 columns at once
+    if (rows == 0) {  // no outputs
+    } else if (!whole) {  // bf16 piece: all 512 columns at once
 #pragma unroll
       for (int ct = 0; ct < 16; ++ct)
 #pragma unroll
@@ -641,7 +680,7 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
                          pack_bf16x2(acc[ct][4 * q + 2] * inv_l, acc[ct][4 * q + 3] * inv_l));
       wide_lds_wait();  // this wave's rows are in LDS
       char* dst = (char*)(p.part_out + ((size_t)(g + b) * H + 32 * wave) * kMlaC);
-      wide_store_rows(dst, kMlaC * 2, stage + 4 * lane, 16 * lane);
+      wide_store_rows(dst, kMlaC * 2, stage + 4 * lane, 16 * lane, rows);
     } else {  // fp32 final: two halves of 256 columns
       char* dst = (char*)(p.out + ((size_t)b * H + 32 * wave) * kMlaC);
 #pragma unroll
@@ -656,7 +695,7 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
                             acc[ct][4 * q + 2] * inv_l, acc[ct][4 * q + 3] * inv_l);
           }
         wide_lds_wait();
-        wide_store_rows(dst, kMlaC * 4, stage + 4 * lane, 1024 * hc + 16 * lane);
+        wide_store_rows(dst, kMlaC * 4, stage + 4 * lane, 1024 * hc + 16 * lane, rows);
         wide_lds_wait();  // the next half overwrites the rows
       }
     }

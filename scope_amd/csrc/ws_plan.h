@@ -24,7 +24,6 @@ struct Plan {
   int T;  // total blocks (the host keeps it below 2^31 / grid)
   int n;  // workgroups with work (min(grid, T)), at most 4096
   int q, r;  // T = q n + r
-  bool seq;  // sequence-aligned ranges (plan_build with s_wpref)
   // The calling split's range [begin, end) and the sequence of block `begin`.
   bool has_work;
   int begin, end, b0;
@@ -34,12 +33,15 @@ struct Plan {
 // DPP sequence: every lane of the wave must be active.
 extern "C" __device__ int __ockl_wfscan_add_i32(int, bool);
 
-// Most sequences the sequence-aligned plan takes.
-constexpr int kSeqPlanMax = 64;
-// Blocks per split the sequence-aligned plan may add over ceil(T / n) and
-// still be chosen: a split whose range enters a second sequence restarts
-// its load stream there, which costs the MLA step about four blocks' time.
-constexpr int kAlignSlack = 3;
+// Most sequences the sequence-aligned plan takes (four a lane).
+constexpr int kSeqPlanMax = 256;
+// Step of the block counts per split the sequence-aligned plan tries over
+// ceil(T / n): up to three steps are accepted.  A split whose range enters a
+// second sequence restarts its load stream there, which costs the 16-head MLA
+// step about four blocks' time and the wide one (queries of 128 heads in, 128
+// KB of outputs out) about ten.
+constexpr int kAlignStep = 1;
+constexpr int kAlignStepWide = 3;
 
 // Workgroup-uniform value moved to a scalar register.
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -77,7 +79,6 @@ __device__ __forceinline__ Plan plan_of(int T, int grid) {
   p.n = min(grid, T);
   p.q = p.n > 0 ? (int)((unsigned)T / (unsigned)p.n) : 0;
   p.r = T - p.q * p.n;
-  p.seq = false;
   p.has_work = false;
   p.begin = p.end = 0;
   p.b0 = -1;
@@ -90,101 +91,157 @@ __device__ __forceinline__ int plan_start(const Plan& p, int g) {
   return g * p.q + (int)((unsigned)(g * p.r) / (unsigned)p.n);
 }
 
-// The sequence-aligned plan's blocks per split: the smallest M in [base,
-// base + kAlignSlack], base = ceil(T / n), at which the sequences (lane b:
-// nb blocks) need at most n splits, or 0 if there is none.  The four
-// candidates are counted in one pass, summed over the wave as 16-bit halves
-// (each count is at most n + 64).  Every lane must call it.
-__device__ __forceinline__ int plan_align(int nb, const Plan& p) {
-  static_assert(kAlignSlack == 3, "four candidates, two per packed sum");
+// Splits of a sequence of nb blocks at M blocks per split (rM = 1 / M): ceil(nb
+// / M), or one more where the product rounds up; at least 1 and at most nb for
+// nb > 0, and the same in every kernel.
+__device__ __forceinline__ int plan_nsplits(int nb, float rM) {
+  return nb > 0 ? (int)((float)(nb - 1) * rM) + 1 : 0;
+}
+
+// The sequence-aligned plan's blocks per split: the first M of base, base +
+// step, base + 2 step, base + 3 step, base = ceil(T / n), at which the
+// sequences (nb: the blocks of a lane's K sequences) need at most n splits, or
+// 0 if there is none.  The four candidates are counted in one pass, summed
+// over the wave as 16-bit halves (each count is at most n + 2 B).  Every lane
+// must call it.
+template <int K>
+__device__ __forceinline__ int plan_align(const int (&nb)[K], const Plan& p, int step) {
   const int base = (p.T + p.n - 1) / p.n;
-  uint32_t c01 = 0, c23 = 0;
-  if (nb > 0) {
-    const uint32_t u = (uint32_t)nb;
-    c01 = (u + base - 1) / base | ((u + base) / (base + 1)) << 16;
-    c23 = (u + base + 1) / (base + 2) | ((u + base + 2) / (base + 3)) << 16;
+  float rM[4];
+  uint32_t cnt[2] = {0, 0};
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    rM[c] = __builtin_amdgcn_rcpf((float)(base + c * step));
+    uint32_t sum = 0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) sum += plan_nsplits(nb[k], rM[c]);
+    cnt[c >> 1] += sum << (16 * (c & 1));
   }
-  c01 = __ockl_wfred_add_u32(c01);
-  c23 = __ockl_wfred_add_u32(c23);
-  const int cnt[4] = {(int)(c01 & 0xffffu), (int)(c01 >> 16), (int)(c23 & 0xffffu),
-                      (int)(c23 >> 16)};
+  cnt[0] = __ockl_wfred_add_u32(cnt[0]);
+  cnt[1] = __ockl_wfred_add_u32(cnt[1]);
   int M = 0;
 #pragma unroll
-  for (int c = kAlignSlack; c >= 0; --c)
-    if (uniform(cnt[c]) <= p.n) M = base + c;
+  for (int c = 3; c >= 0; --c)
+    if (uniform((cnt[c >> 1] >> (16 * (c & 1))) & 0xffffu) <= p.n) M = base + c * step;
   return M;
+}
+
+// plan_build for at most 64 K sequences, K consecutive ones a lane.
+template <int K>
+__device__ __forceinline__ Plan plan_build_k(const int32_t* len_in, int add, int cap, int B, int R,
+                                             int grid, int* s_pref, int* s_len, int g, int ng,
+                                             int step) {
+  const int lane = threadIdx.x & 63;
+  const int v0 = K * lane;
+  int l[K], nb[K], sum = 0;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    l[k] = K > 1 || lane < B ? plan_len(len_in, seq_of(min(v0 + k, B - 1), ng), add, cap) : 0;
+    if (v0 + k >= B) l[k] = 0;
+  }
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    nb[k] = R * ((l[k] + 31) >> 5);
+    sum += nb[k];
+  }
+  const int incl = __ockl_wfscan_add_i32(sum, true);
+  int run = incl - sum;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    if (v0 + k < B) {
+      s_pref[v0 + k] = run;
+      s_len[v0 + k] = l[k];
+    }
+    run += nb[k];
+  }
+  const int T = __builtin_amdgcn_readlane(incl, 63);
+  if (lane == 0) s_pref[B] = T;
+  Plan p = plan_of(T, grid);
+  const int M = R == 1 && B >= 2 && p.n > 0 ? plan_align<K>(nb, p, step) : 0;
+  if (M > 0) {
+    const float rM = __builtin_amdgcn_rcpf((float)M);
+    int ns[K], nsum = 0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      ns[k] = plan_nsplits(nb[k], rM);
+      nsum += ns[k];
+    }
+    const int w = __ockl_wfscan_add_i32(nsum, true);
+    if (g >= 0 && g < __builtin_amdgcn_readlane(w, 63)) {
+      // split g: its lane (the first with w > g), the lane's sequence and the
+      // split's number j of that sequence's
+      const int at = __builtin_ctzll(__builtin_amdgcn_ballot_w64(w > g));
+      int j = g - __builtin_amdgcn_readlane(w - nsum, at);
+      int first = __builtin_amdgcn_readlane(incl - sum, at);
+      int nbb = __builtin_amdgcn_readlane(nb[0], at);
+      int nsb = __builtin_amdgcn_readlane(ns[0], at);
+      p.b0 = K * at;
+#pragma unroll
+      for (int k = 1; k < K; ++k) {
+        const int nbk = __builtin_amdgcn_readlane(nb[k], at);
+        const int nsk = __builtin_amdgcn_readlane(ns[k], at);
+        if (p.b0 == K * at + k - 1 && j >= nsb) {
+          j -= nsb;
+          first += nbb;
+          nbb = nbk;
+          nsb = nsk;
+          p.b0 = K * at + k;
+        }
+      }
+      p.has_work = true;
+      p.begin = first + j * nbb / nsb;
+      p.end = first + (j + 1) * nbb / nsb;
+    }
+    return p;
+  }
+  if (g >= 0 && g < p.n) {
+    p.has_work = true;
+    p.begin = plan_start(p, g);
+    p.end = plan_start(p, g + 1);
+    // the lane of the first sequence that ends past block `begin`, and which
+    const int at = __builtin_ctzll(__builtin_amdgcn_ballot_w64(incl > p.begin));
+    int last = __builtin_amdgcn_readlane(incl - sum, at);
+    p.b0 = K * at;
+#pragma unroll
+    for (int k = 0; k + 1 < K; ++k) {
+      last += __builtin_amdgcn_readlane(nb[k], at);
+      if (last <= p.begin) p.b0 = K * at + k + 1;
+    }
+  }
+  return p;
 }
 
 // Builds s_pref[0..B] (exclusive prefix of blocks per sequence, R rows each)
 // and the lengths s_len[0..B) (plan_len), and returns the plan.  Every wave
 // of the workgroup calls it with all its lanes, builds the whole plan by
-// itself (lane b: sequence b; above 64 sequences, ceil(B / 64) consecutive
+// itself (B <= 64: lane b is sequence b; above, ceil(B / 64) consecutive
 // ones a lane) and writes the same values, reading back only what it wrote:
 // no barrier between the kernel start and its first loads.  (With more than
 // 64 sequences built together by the workgroup, behind three barriers and a
 // chain of one load per sequence of a lane, GQA B = 256 took 204.7 us a step,
 // against 187.5 with every wave on its own here and in the merge.)
 //
-// With one row per sequence (R == 1) and 2 to 64 sequences, the plan may
-// instead be sequence-aligned: sequence b gets n_b = ceil(nb(b) / M) splits, M
-// the smallest block count per split with sum_b n_b <= n, which take equal
-// shares of its blocks, so no split spans two sequences.  It is chosen when
-// M <= ceil(T / n) + kAlignSlack (seq set, s_wpref[b] = first split of
-// sequence b, s_wpref[B] = splits used; kSeqPlanMax + 1 ints).  Every kernel
-// of a call (step and merge) passes the same arguments and so makes the same
-// choice.
+// With one row per sequence (R == 1) and 2 to kSeqPlanMax sequences, the plan
+// may instead be sequence-aligned: sequence b gets n_b = plan_nsplits(nb(b), M)
+// splits, M the first block count per split of plan_align with sum_b n_b <= n,
+// which take equal shares of its blocks, so no split spans two sequences.
+// Every kernel of a call (step and merge) passes the same arguments and so
+// makes the same choice.
 //
 // Split g (g >= 0) gets its range in has_work / begin / end and the sequence
 // of its first block in b0.
 //
 // ng > 1: B counts plan sequences v = b ng + group, whose lengths are
-// len_in[v / ng] (seq_of).
+// len_in[v / ng] (seq_of).  step: kAlignStep or kAlignStepWide.
 __device__ __forceinline__ Plan plan_build(const int32_t* len_in, int add, int cap, int B, int R,
-                                           int grid, int* s_pref, int* s_len, int* s_wpref,
-                                           int g, int ng) {
-  const int lane = threadIdx.x & 63;
-  if (__builtin_expect(B >= 1 && B <= 64, 1)) {
-    const int l = lane < B ? plan_len(len_in, seq_of(lane, ng), add, cap) : 0;
-    const int nb = R * ((l + 31) >> 5);
-    const int incl = __ockl_wfscan_add_i32(nb, true);
-    if (lane < B) {
-      s_pref[lane] = incl - nb;
-      s_len[lane] = l;
-    }
-    const int T = __builtin_amdgcn_readlane(incl, B - 1);
-    if (lane == 0) s_pref[B] = T;
-    Plan p = plan_of(T, grid);
-    const int M = R == 1 && B >= 2 && p.n > 0 ? plan_align(nb, p) : 0;
-    if (M > 0) {
-      const int ns = nb > 0 ? (nb + M - 1) / M : 0;
-      const int w = __ockl_wfscan_add_i32(ns, true);
-      const int used = __builtin_amdgcn_readlane(w, B - 1);
-      if (lane < B) s_wpref[lane] = w - ns;
-      if (lane == 0) s_wpref[B] = used;
-      p.seq = true;
-      if (g >= 0 && g < used) {
-        // split g: sequence b (the first with w > g), its j-th of ns splits
-        const int b = __builtin_ctzll(__builtin_amdgcn_ballot_w64(lane < B && w > g));
-        const int j = g - (__builtin_amdgcn_readlane(w, b) - __builtin_amdgcn_readlane(ns, b));
-        const int nsb = __builtin_amdgcn_readlane(ns, b);
-        const int first = __builtin_amdgcn_readlane(incl, b) - __builtin_amdgcn_readlane(nb, b);
-        const int nbb = __builtin_amdgcn_readlane(nb, b);
-        p.has_work = true;
-        p.begin = first + j * nbb / nsb;
-        p.end = first + (j + 1) * nbb / nsb;
-        p.b0 = b;
-      }
-      return p;
-    }
-    if (g >= 0 && g < p.n) {
-      p.has_work = true;
-      p.begin = plan_start(p, g);
-      p.end = plan_start(p, g + 1);
-      p.b0 = __builtin_ctzll(__builtin_amdgcn_ballot_w64(lane < B && incl > p.begin));
-    }
-    return p;
-  }
+                                           int grid, int* s_pref, int* s_len, int g, int ng,
+                                           int step) {
+  if (__builtin_expect(B >= 1 && B <= 64, 1))
+    return plan_build_k<1>(len_in, add, cap, B, R, grid, s_pref, s_len, g, ng, step);
+  if (B <= kSeqPlanMax)
+    return plan_build_k<4>(len_in, add, cap, B, R, grid, s_pref, s_len, g, ng, step);
   // lane: sequences c * lane .. c * lane + c - 1, four loads at a time
+  const int lane = threadIdx.x & 63;
   const int c = (B + 63) >> 6;
   const int v0 = c * lane;
   int sum = 0;
@@ -246,7 +303,8 @@ struct RowSplits {
 // Every lane of the wave must be active; v and r are wave-uniform.
 template <int K>
 __device__ __forceinline__ RowSplits plan_row_k(const int32_t* len_in, int add, int cap, int B,
-                                                int R, int grid, int v, int r, int ng) {
+                                                int R, int grid, int v, int r, int ng,
+                                                int step) {
   const int lane = threadIdx.x & 63;
   int nb[K];
   uint32_t sum = 0, before = 0;
@@ -263,11 +321,14 @@ __device__ __forceinline__ RowSplits plan_row_k(const int32_t* len_in, int add, 
   }
   if (rs.nbb == 0) return rs;
   const Plan p = plan_of(R * uniform((int)__ockl_wfred_add_u32(sum)), grid);
-  const int M = K == 1 && R == 1 && B >= 2 ? plan_align(nb[0], p) : 0;
+  const int M = R == 1 && B >= 2 ? plan_align<K>(nb, p, step) : 0;
   if (M > 0) {
-    rs.w_first =
-        uniform((int)__ockl_wfred_add_u32(lane < v ? ((uint32_t)nb[0] + M - 1) / M : 0u));
-    rs.nseg = (rs.nbb + M - 1) / M;
+    const float rM = __builtin_amdgcn_rcpf((float)M);
+    uint32_t ns = 0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) ns += lane + 64 * k < v ? plan_nsplits(nb[k], rM) : 0;
+    rs.w_first = uniform((int)__ockl_wfred_add_u32(ns));
+    rs.nseg = uniform(plan_nsplits(rs.nbb, rM));
   } else {
     const int start = R * uniform((int)__ockl_wfred_add_u32(before)) + r * rs.nbb;
     rs.w_first = plan_owner(p, start);
@@ -276,9 +337,10 @@ __device__ __forceinline__ RowSplits plan_row_k(const int32_t* len_in, int add, 
   return rs;
 }
 __device__ __forceinline__ RowSplits plan_row(const int32_t* len_in, int add, int cap, int B,
-                                              int R, int grid, int v, int r, int ng) {
-  if (B <= 64) return plan_row_k<1>(len_in, add, cap, B, R, grid, v, r, ng);
-  if (B <= 256) return plan_row_k<4>(len_in, add, cap, B, R, grid, v, r, ng);
+                                              int R, int grid, int v, int r, int ng,
+                                              int step) {
+  if (B <= 64) return plan_row_k<1>(len_in, add, cap, B, R, grid, v, r, ng, step);
+  if (B <= kSeqPlanMax) return plan_row_k<4>(len_in, add, cap, B, R, grid, v, r, ng, step);
   const int lane = threadIdx.x & 63;
   uint32_t sum = 0, before = 0;
 #pragma unroll 4

@@ -20,6 +20,7 @@
 #pragma once
 
 #include "ws_common.h"
+#include "ws_plan.h"
 
 namespace ws {
 
@@ -50,25 +51,37 @@ __host__ __device__ inline SplitWorkspace carve_workspace(void* base, int rows_k
 }
 
 // Layout of an absorbed-MLA call with B sequences of H heads (H a multiple
-// of 16).  H = 128 over at most 64 sequences (DeepSeek-V2) runs the wide
-// kernel (ws_mla_wide.h): its plan sequences are the sequences and a piece
-// holds all 128 heads.  Other head counts plan (sequence, 16-head group)
-// pairs with 16-head pieces.  The step, the merges and the workspace query of
-// a call all take their layout from here, so they agree.
-constexpr int kWideHeads = 128;
-constexpr int kWideMaxSeqs = 64;
+// of 16).  The wide kernel (ws_mla_wide.h) reads a latent block once for up to
+// 128 heads; its plan sequences are the sequences and a piece holds all H
+// heads.  Other calls plan (sequence, 16-head group) pairs with 16-head pieces
+// and read a block once per group.  The step, the merges and the workspace
+// query of a call all take their layout from here, so they agree.
+//
+// 128 heads always run wide.  Fewer do from B * H = 1024 on (in front of that
+// line the wide kernel's longer start and end cost more than the repeated
+// reads).  Step kernel with its reduce, group layout -> wide, ragged lengths up
+// to the given one: B 32 x H 32: 300 tokens 23.4 -> 21.2 us, 4k 53.7 -> 42.3;
+// B 16 x H 64: 300 tokens 23.5 -> 20.8, 16k 140 -> 62; B 11 x H 96: 300 tokens
+// 26.4 -> 21.3, 16k 148 -> 55.  Below it: B 16 x H 32 of 1000 tokens 19.1 ->
+// 21.5, B 8 x H 64 of 2048 23.2 -> 26.3.
+constexpr int kWideHeads = 128;    // heads of the wide kernel's four waves
+constexpr int kWideMinHeads = 32;
+constexpr int kWideMinRows = 1024;  // B * H from which fewer than 128 heads run it
+constexpr int kWideMaxSeqs = 16 * kMaxSeqs / kWideMinHeads;  // (a call takes B * H / 16 <= kMaxSeqs)
 struct MlaLayout {
   bool wide;
   int ng;           // plan sequences per sequence
   int piece_heads;  // heads of one piece
   int plan_seqs;    // B * ng
+  int step;         // the plan's alignment step (ws_plan.h)
 };
 __host__ __device__ inline MlaLayout mla_layout(int B, int H) {
   MlaLayout l;
-  l.wide = H == kWideHeads && B >= 1 && B <= kWideMaxSeqs;
+  l.wide = H == kWideHeads || (H >= kWideMinHeads && H < kWideHeads && (long long)B * H >= kWideMinRows);
   l.ng = l.wide ? 1 : H / 16;
   l.piece_heads = l.wide ? H : 16;
   l.plan_seqs = B * l.ng;
+  l.step = l.wide ? kAlignStepWide : kAlignStep;
   return l;
 }
 

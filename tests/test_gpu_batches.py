@@ -1,5 +1,5 @@
 """Batches of many sequences on the GPU: the plan's limits (64 sequences, one
-per lane; 256, four per lane; above, the workgroup's plan), rows cut over
+per lane; 256, four per lane; above, more), rows cut over
 splits and rows held whole, empty sequences among them, through the finished
 partial, the split step with a host partial and its merge, and the W_UV
 epilogue.  Against fp64 over the same bf16 inputs.
@@ -95,7 +95,10 @@ def test_gqa_many_sequences(B, Hkv, G, wg):
 
 
 @pytest.mark.parametrize("B,H,wg", [(65, 16, 0), (200, 16, 0), (257, 16, 40), (100, 32, 0),
-                                    (65, 128, 0), (96, 128, 300), (140, 128, 9), (256, 128, 0)])
+                                    (65, 128, 0), (96, 128, 300), (140, 128, 9), (256, 128, 0),
+                                    # one pass for all heads (B * H >= 1024) and its edges
+                                    (31, 32, 0), (32, 32, 0), (1024, 32, 0), (22, 48, 7),
+                                    (16, 64, 0), (64, 80, 300), (11, 96, 0), (10, 112, 5)])
 def test_mla_many_sequences(B, H, wg):
     lens = _lens(B, B + H, 2500)
     scale = 192 ** -0.5
