@@ -622,11 +622,10 @@ static int gqa_launch(const uint16_t* q, const uint16_t* k_new, const uint16_t* 
   int rc = check_launch(name);
   if (rc != WS_OK || !combine) return rc;
   // One-launch entry points: the rows held by several waves are combined by
-  // the split merge on the same stream, in place (each element is read and
-  // written by the same thread; the merge workgroups of a row's column chunks
-  // all write its unchanged lse when one wave held it).
-  rc = merge_split_pieces(len_in, k_new ? 1 : 0, B, Hkv, G, D, prm.cap, n, out, lse, prm.ws,
-                          out, lse, out_bf16, s);
+  // the split merge on the same stream.
+  const MlaLayout lay = {false, 1, G, B, kAlignStep};
+  rc = merge_split_pieces(len_in, k_new ? 1 : 0, lay, Hkv, G, D, prm.cap, n, out, lse, prm.ws,
+                          out_bf16, s);
   return rc != WS_OK ? rc : check_launch(name);
 }
 

@@ -5,6 +5,8 @@
 // needed after its host-to-device copy.
 #include <math.h>
 
+#include <algorithm>
+
 #include "ws_plan.h"
 #include "ws_reduce.h"
 
@@ -88,20 +90,32 @@ __global__ __launch_bounds__(128) void lse_merge_kernel(
 // ---------------------------------------------------------------------------
 // Split combine + host merge of a deferred-combine decode step.
 //
-// One 64-lane workgroup per output row (kv row * heads + head) and 256-column
-// chunk.  It rebuilds
-// the step's plan from the post-step lengths (ws_plan.h) to find the row's
-// GPU pieces: the final (out, lse) the step wrote when one workgroup held the
-// row, else the partials of the row's workgroups (slots w + kv row), then
-// LSE-combines them with the host partial (format FMT, or none when FMT < 0)
-// and writes the normalised result.  Runs after the step on the same stream,
-// so plain loads see its writes.
+// It rebuilds the step's plan from the post-step lengths (ws_plan.h) to find
+// the GPU pieces of a plan row (kv row): the final (out, lse) the step wrote
+// when one workgroup held the row, else the partials of the row's workgroups
+// (slots w + kv row), then LSE-combines them with the host partial (format FMT,
+// or none when FMT < 0) and writes the normalised result.  Runs after the step
+// on the same stream, so plain loads see its writes.
+//
+// A wave owns a group of up to 64 float4 columns: the whole output rows (heads)
+// of the plan row that fit, or a part of one row wider than 256.  What bounds a
+// merge is the chain of round trips (lengths, then pieces) and, for rows of
+// many pieces, how many piece loads are in flight.  So the lse values travel
+// with the pieces' columns (piece_batch keeps running weights; no pass over
+// the lse values first), and PS waves share a column group, wave i taking
+// pieces i, i + PS, ... and the first combining them through LDS.  With few
+// pieces a row (PS = 1) a wave walks several groups of its plan row on one plan.
+//   (weights first, one wave a row and 256 columns: 32 rows of 64 pieces x 128
+//   columns 6.8 us, 128 rows of 32 pieces x 512 columns 6.0, 12288 rows of two
+//   to three pieces and a host partial x 512 columns 30, 8192 rows of one piece
+//   x 128 columns 25.0; now 4.7, 4.6, 25.5 and 7.1)
 struct MergeSplitParams {
   const int32_t* gpu_len;
   // B: plan sequences; ng > 1 for absorbed MLA with H = 16 ng heads, whose
   // plan sequences are (sequence, 16-head group) pairs (ws_plan.h seq_of).
   int B, ng, R, heads, Dv, cap, grid;
-  int step;  // the plan's alignment step
+  int step;       // the plan's alignment step
+  bool in_place;  // out_g / lse_g are the outputs: rows of one piece stay as they are
   int add;  // lengths are gpu_len[b] + add (1 when gpu_len is a fused step's len_in)
   const float* out_g;
   const float* lse_g;
@@ -115,99 +129,170 @@ struct MergeSplitParams {
   float* lse_out;
 };
 
-// LDS of a merge: one weight per piece a row can have (a row's pieces come from
-// different splits).  Sized by the call, not by the most a call may have: 16
-// KB kept a CU to nine of these one-wave workgroups.
-static size_t merge_lds(int n) { return 4 * (size_t)n; }
+// Waves that share a column group: 1, or more where the rows have many pieces
+// on average (n splits over rows plan rows, about n / rows + 1 each) and the
+// column groups alone do not fill the chip: with eight waves on each of 1024
+// groups of 64 pieces (4 sequences x 128 heads x 512 columns) the merge took
+// 11.0 us, with one 9.4; on 16 groups of 64 pieces 4.6 against 6.8.
+constexpr int kMergeMaxStreams = 8;
+static int merge_streams(int n, long long rows, int groups) {
+  if (n >= 24 * rows && rows * groups <= 512) return kMergeMaxStreams;
+  return n >= 4 * rows && rows * groups <= 1024 ? 4 : 1;
+}
+// Waves of a merge launch with PS = 1 (32 a CU); further groups are walked.
+constexpr long long kMergeWaves = 8192;
+constexpr int kMergeWgWaves = 4;
 
-// One 64-lane workgroup per (output row, 256-column chunk): lane t owns float4
-// column chunk * 64 + t and accumulates it over the pieces with eight loads
-// in flight.
-constexpr int kMergeChunk4 = 64;
+// A thread's place in column group `grp` of a plan row: head h of the row and
+// float4 column c of the head (ok: inside the row).
+struct MergeCol {
+  int h, c;
+  bool ok;
+};
+__device__ __forceinline__ MergeCol merge_col(int grp, int lane, int heads, int Dv4) {
+  MergeCol m;
+  if (Dv4 <= 64) {  // 64 / Dv4 whole rows
+    const int per = 64 / Dv4;
+    const int r = lane / Dv4;
+    m.h = grp * per + r;
+    m.c = lane - r * Dv4;
+    m.ok = r < per && m.h < heads;
+  } else {
+    const int parts = (Dv4 + 63) >> 6;
+    m.h = grp / parts;
+    m.c = 64 * (grp - m.h * parts) + lane;
+    m.ok = m.c < Dv4;
+  }
+  if (!m.ok) {
+    m.h = min(m.h, heads - 1);
+    m.c = 0;
+  }
+  return m;
+}
+__host__ __device__ inline int merge_groups(int heads, int Dv4) {
+  return Dv4 <= 64 ? (heads + 64 / Dv4 - 1) / (64 / Dv4) : heads * ((Dv4 + 63) >> 6);
+}
 
-template <int FMT>
-__global__ __launch_bounds__(64) void merge_split_kernel(const MergeSplitParams p) {
-  extern __shared__ float s_w[];  // weights of the row's pieces (at most p.grid)
-  const int qrow = blockIdx.x;
-  const int t = threadIdx.x;
-  const int krow = qrow / p.heads;
-  const int h = qrow - krow * p.heads;
-  const int b = krow / p.R;
-  const int r = krow - b * p.R;
-  // The host partial's address depends on nothing the plan computes: its
-  // loads go out first.
-  const int c = blockIdx.y * kMergeChunk4 + t;  // float4 column
-  const bool col_ok = c < (p.Dv >> 2);
-  float lb = neg_inf();
-  float4 ob = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (FMT >= 0)
-    load_b<(FMT >= 0 ? FMT : 0)>(p.b_out, p.b_aux0, p.b_aux1, qrow, p.Dv, col_ok ? c : 0, lb,
-                                 ob);
-  const RowSplits rs = plan_row(p.gpu_len, p.add, p.cap, p.B, p.R, p.grid, b, r, p.ng, p.step);
-  // One piece: the step's final partial (out_g, fp32); several: their bf16
-  // workspace slots, piece s at pieces + s * sstride.
-  int n = 1;
-  const float* src = p.out_g + (size_t)qrow * p.Dv;
-  const uint16_t* pieces = nullptr;
-  const float* lsrc = p.lse_g + qrow;  // lse of piece s at lsrc[s * lstride]
-  size_t sstride = 0, lstride = 0;
+// What stream `st` of PS adds to the row's output: its share of the pieces, or
+// (the first stream) the final partial of a row that one split held.
+__device__ __forceinline__ PieceAcc merge_stream(const MergeSplitParams& p, const RowSplits& rs,
+                                                 size_t krow, int h, int c, int heads, int st,
+                                                 int PS) {
   if (rs.nseg > 1) {
-    n = rs.nseg;
-    const size_t slot0 = (size_t)(rs.w_first + krow) * p.heads + h;
-    pieces = p.part_out + slot0 * p.Dv;
-    lsrc = p.part_lse + slot0;
-    sstride = (size_t)p.heads * p.Dv;
-    lstride = p.heads;
+    const size_t slot0 = ((size_t)rs.w_first + krow) * heads + h;
+    return piece_stream(p.part_out + slot0 * p.Dv + 4 * c, (size_t)heads * p.Dv,
+                        p.part_lse + slot0, heads, st, PS, rs.nseg);
   }
-  // The pieces' columns are requested with their lse values.
-  const int cc = col_ok ? c : 0;
-  uint2 pv[8];
-  float4 v1 = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (!pieces)
-    v1 = ((const float4*)src)[cc];
-  else if (n <= 8)
-    preload_pieces(pieces + 4 * cc, sstride, n, pv);
-  // weights: M over the GPU pieces and the host partial
-  float mx = lb;
-  for (int s = t; s < n; s += 64) {
-    const float v = lsrc[(size_t)s * lstride];
-    s_w[s] = v;
-    mx = max_nan(mx, v);
+  PieceAcc x = piece_acc_empty();
+  if (st == 0) {
+    const size_t q = krow * heads + h;
+    const float4 v = ((const float4*)(p.out_g + q * p.Dv))[c];
+    x.m = p.lse_g[q];
+    if (x.m != neg_inf()) {
+      x.sum = 1.f;
+      x.a = v;
+    }
   }
-  for (int o = 1; o < 64; o <<= 1) mx = max_nan(mx, __shfl_xor(mx, o));
-  float sum = 0.f;
-  for (int s = t; s < n; s += 64) {
-    const float w = mx == neg_inf() ? 0.f : __expf(s_w[s] - mx);
-    s_w[s] = w;
-    sum += w;
-  }
-  for (int o = 1; o < 64; o <<= 1) sum += __shfl_xor(sum, o);
-  const float wb = (FMT >= 0 && mx != neg_inf()) ? __expf(lb - mx) : 0.f;
-  const float L = sum + wb;
-  __syncthreads();
-  const float inv = L == 0.f ? 0.f : 1.f / L;
-  if (blockIdx.y == 0 && t == 0 && p.lse_out)
-    p.lse_out[qrow] = L == 0.f ? neg_inf() : mx + __logf(L);
-  if (!col_ok) return;
+  return x;
+}
+
+// The finished row's columns from n accumulators acc(i) and the host partial
+// (lb, ob): the output in o and the row's lse.
+template <class F>
+__device__ __forceinline__ void merge_finish(const F& acc, int n, float lb, const float4& ob,
+                                             float4& o, float& lse) {
+  float M = lb;
+  for (int i = 0; i < n; ++i) M = fmaxf(M, acc(i).m);
+  const float wb = piece_weight(lb, M);
   // an empty host side has weight 0 and must not turn its output into NaN
   float4 a = wb > 0.f ? make_float4(wb * ob.x, wb * ob.y, wb * ob.z, wb * ob.w)
                       : make_float4(0.f, 0.f, 0.f, 0.f);
-  if (pieces) {
-    if (n <= 8)
-      accum_preloaded(pv, n, s_w, a);
-    else
-      accum_pieces(pieces + 4 * c, sstride, n, s_w, a);
-  } else {
-    const float w = s_w[0];
-    a.x += w * v1.x; a.y += w * v1.y; a.z += w * v1.z; a.w += w * v1.w;
+  float L = wb;
+  for (int i = 0; i < n; ++i) {
+    const PieceAcc x = acc(i);
+    const float f = acc_factor(x.m, M);
+    L += x.sum * f;
+    a.x += x.a.x * f; a.y += x.a.y * f; a.z += x.a.z * f; a.w += x.a.w * f;
   }
-  const float4 o = make_float4(a.x * inv, a.y * inv, a.z * inv, a.w * inv);
-  if (p.out_f32) ((float4*)(p.out_f32 + (size_t)qrow * p.Dv))[c] = o;
-  if (p.out_bf16) {
-    uint2 packed;
-    packed.x = pack_bf16x2(o.x, o.y);
-    packed.y = pack_bf16x2(o.z, o.w);
-    ((uint2*)(p.out_bf16 + (size_t)qrow * p.Dv))[c] = packed;
+  const float inv = L == 0.f ? 0.f : 1.f / L;
+  o = make_float4(a.x * inv, a.y * inv, a.z * inv, a.w * inv);
+  lse = L == 0.f ? neg_inf() : M + __logf(L);
+}
+
+template <int FMT, int PS>
+__global__ __launch_bounds__(64 * (PS > kMergeWgWaves ? PS : kMergeWgWaves)) void
+merge_split_kernel(const MergeSplitParams p) {
+  __shared__ PieceAcc s_acc[PS > 1 ? PS : 1][64];
+  const int lane = threadIdx.x & 63;
+  const int wave = uniform(threadIdx.x >> 6);
+  const size_t krow = blockIdx.x;
+  const int b = uniform(blockIdx.x / p.R);
+  const int r = blockIdx.x - b * p.R;
+  const int Dv4 = p.Dv >> 2;
+  const int groups = merge_groups(p.heads, Dv4);
+  const int waves = blockDim.x >> 6;
+  int grp = PS > 1 ? blockIdx.y : blockIdx.y * waves + wave;
+  if (PS == 1 && grp >= groups) return;
+  // The host partial's address depends on nothing the plan computes: its
+  // loads go out first.
+  MergeCol mc = merge_col(grp, lane, p.heads, Dv4);
+  float lb = neg_inf();
+  float4 ob = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto host = [&]() {
+    if (FMT >= 0)
+      load_b<(FMT >= 0 ? FMT : 0)>(p.b_out, p.b_aux0, p.b_aux1, (int)(krow * p.heads + mc.h),
+                                   p.Dv, mc.c, lb, ob);
+  };
+  host();
+  const RowSplits rs = plan_row(p.gpu_len, p.add, p.cap, p.B, p.R, p.grid, b, r, p.ng, p.step);
+  if (p.in_place && rs.nseg <= 1) return;  // out / lse hold the row
+  auto store = [&](const float4& o, float lse) {
+    if (!mc.ok) return;
+    const size_t q = krow * p.heads + mc.h;
+    if (p.out_f32) ((float4*)(p.out_f32 + q * p.Dv))[mc.c] = o;
+    if (p.out_bf16)
+      ((uint2*)(p.out_bf16 + q * p.Dv))[mc.c] =
+          make_uint2(pack_bf16x2(o.x, o.y), pack_bf16x2(o.z, o.w));
+    if (p.lse_out && mc.c == 0) p.lse_out[q] = lse;
+  };
+  float4 o;
+  float lse;
+  if constexpr (PS > 1) {
+    s_acc[wave][lane] = merge_stream(p, rs, krow, mc.h, mc.c, p.heads, wave, PS);
+    __syncthreads();
+    if (wave != 0) return;
+    merge_finish([&](int i) { return s_acc[i][lane]; }, PS, lb, ob, o, lse);
+    store(o, lse);
+  } else {
+    for (;;) {
+      const PieceAcc x = merge_stream(p, rs, krow, mc.h, mc.c, p.heads, 0, 1);
+      merge_finish([&](int) { return x; }, 1, lb, ob, o, lse);
+      store(o, lse);
+      grp += waves * gridDim.y;
+      if (grp >= groups) break;
+      mc = merge_col(grp, lane, p.heads, Dv4);
+      host();
+    }
+  }
+}
+
+// Launches merge_split_kernel<FMT> over rows plan rows.
+template <int FMT>
+static void launch_merge(const MergeSplitParams& p, long long rows, hipStream_t s) {
+  const int groups = merge_groups(p.heads, p.Dv / 4);
+  const int PS = merge_streams(p.grid, rows, groups);
+  if (PS == kMergeMaxStreams) {
+    hipLaunchKernelGGL((merge_split_kernel<FMT, kMergeMaxStreams>),
+                       dim3((unsigned)rows, groups), dim3(64 * kMergeMaxStreams), 0, s, p);
+  } else if (PS == 4) {
+    hipLaunchKernelGGL((merge_split_kernel<FMT, 4>), dim3((unsigned)rows, groups), dim3(256), 0, s,
+                       p);
+  } else {
+    const int waves = std::min(groups, kMergeWgWaves);
+    const long long fit = std::max(kMergeWaves / (rows * waves), 1LL);
+    const int wgs = (int)std::min<long long>((groups + waves - 1) / waves, fit);
+    hipLaunchKernelGGL((merge_split_kernel<FMT, 1>), dim3((unsigned)rows, wgs), dim3(64 * waves), 0,
+                       s, p);
   }
 }
 
@@ -217,33 +302,34 @@ __global__ __launch_bounds__(64) void merge_split_kernel(const MergeSplitParams 
 // is normalised, rounded to bf16 as the reference rounds it before its bmm,
 // and projected onto W_UV[h] ([Dout][512] bf16), giving out_v[b][h * Dout + v].
 //
-// One 256-thread workgroup per (b, h) row: threads 0..127 merge one float4
-// column each (the same pieces, weights and accumulation order as
-// merge_split_kernel, so the optional latent output is bit-identical to it)
-// into an LDS row; then eight lanes per W_UV row read it 128 contiguous bytes
-// at a time and reduce by shuffles, 32 rows per pass.  W_UV[h] is shared by
-// the B rows of head h through L2.
+// One 256-thread workgroup per (b, h) row: the waves merge its two column groups
+// as merge_split_kernel does (the same streams in the same order, so the
+// optional latent output is bit-identical to it), two waves a group, into an
+// LDS row; then eight lanes per W_UV row read it 128 contiguous bytes at a time
+// and reduce by shuffles, 32 rows per pass.  W_UV[h] is shared by the B rows
+// of head h through L2.
 constexpr int kUvThreads = 256;
 constexpr int kUvGroup = 2;  // passes of 32 W_UV rows whose loads are in flight together
 
-template <int FMT>
+template <int FMT, int PS>
 __global__ __launch_bounds__(kUvThreads) void merge_split_uv_kernel(
     const MergeSplitParams p, const uint16_t* __restrict__ w_uv, int Dout,
     uint16_t* __restrict__ out_v) {
-  extern __shared__ float s_w[];  // weights of the row's pieces (at most p.grid)
-  __shared__ float s_row[512];
-  __shared__ float s_ml[2];  // M, 1 / L
+  constexpr int Dv = 512;
+  constexpr int kGroupWaves = kUvThreads / 128;  // waves of a column group
+  __shared__ PieceAcc s_acc[PS > 1 ? PS : 1][Dv / 4];
+  __shared__ float s_row[Dv];
   const int qrow = blockIdx.x;  // b * heads + h
   const int t = threadIdx.x;
   const int b = qrow / p.heads;
   const int h = qrow - b * p.heads;
-  const int hp = p.heads / p.ng;  // heads of a piece: 16, or 128 (wide layout)
+  const int hp = p.heads / p.ng;  // heads of a piece: 16, or all (wide layout)
   const int pv_seq = qrow / hp;   // plan sequence (b, head group) and head in it
   const int h16 = qrow - pv_seq * hp;
   // The W_UV rows of the first kUvGroup passes do not depend on the merge:
   // their loads go out first and land while the plan and the merge run.
   const int lane8 = t & 7;
-  const int rsub = t >> 3;  // 32 rows per pass
+  const int rsub = t >> 3;  // kUvThreads / 8 rows per pass
   u32x4 wv[kUvGroup][8];
 #pragma unroll
   for (int g = 0; g < kUvGroup; ++g) {
@@ -253,79 +339,33 @@ __global__ __launch_bounds__(kUvThreads) void merge_split_uv_kernel(
     for (int j = 0; j < 8; ++j) wv[g][j] = wrow[j * 8 + lane8];
   }
   // So do the host partial's.
-  const int c = t;  // float4 column (threads < 128)
-  const bool merging = c < (p.Dv >> 2);
+  const int c = t & (Dv / 4 - 1);    // float4 column
+  const int first = uniform(t / (Dv / 4));  // the first stream of this wave
   float lb = neg_inf();
   float4 ob = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (FMT >= 0 && merging)
-    load_b<(FMT >= 0 ? FMT : 0)>(p.b_out, p.b_aux0, p.b_aux1, qrow, p.Dv, c, lb, ob);
+  if (FMT >= 0 && first == 0)
+    load_b<(FMT >= 0 ? FMT : 0)>(p.b_out, p.b_aux0, p.b_aux1, qrow, Dv, c, lb, ob);
   const RowSplits rs = plan_row(p.gpu_len, p.add, p.cap, p.B, 1, p.grid, pv_seq, 0, p.ng, p.step);
-  int n = 1;
-  const float* src = p.out_g + (size_t)qrow * p.Dv;
-  const uint16_t* pieces = nullptr;
-  const float* lsrc = p.lse_g + qrow;
-  size_t sstride = 0, lstride = 0;
-  if (rs.nseg > 1) {  // pieces hold hp heads each
-    n = rs.nseg;
-    const size_t slot0 = (size_t)(rs.w_first + pv_seq) * hp + h16;
-    pieces = p.part_out + slot0 * p.Dv;
-    lsrc = p.part_lse + slot0;
-    sstride = (size_t)hp * p.Dv;
-    lstride = hp;
-  }
-  // The merging threads' piece columns are requested with the lse values.
-  uint2 pv[8];
-  float4 v1 = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (merging) {
-    if (!pieces)
-      v1 = ((const float4*)src)[c];
-    else if (n <= 8)
-      preload_pieces(pieces + 4 * c, sstride, n, pv);
-  }
-  if (t < 64) {  // wave 0: the pieces' weights
-    float mx = lb;
-    for (int s = t; s < n; s += 64) {
-      const float v = lsrc[(size_t)s * lstride];
-      s_w[s] = v;
-      mx = max_nan(mx, v);
+  PieceAcc x;
+#pragma unroll
+  for (int i = 0; i < PS; i += kGroupWaves)
+    if (first + i < PS) {
+      x = merge_stream(p, rs, pv_seq, h16, c, hp, first + i, PS);
+      if (PS > 1) s_acc[first + i][c] = x;
     }
-    for (int o = 1; o < 64; o <<= 1) mx = max_nan(mx, __shfl_xor(mx, o));
-    float sum = 0.f;
-    for (int s = t; s < n; s += 64) {
-      const float w = mx == neg_inf() ? 0.f : __expf(s_w[s] - mx);
-      s_w[s] = w;
-      sum += w;
-    }
-    for (int o = 1; o < 64; o <<= 1) sum += __shfl_xor(sum, o);
-    const float wb = (FMT >= 0 && mx != neg_inf()) ? __expf(lb - mx) : 0.f;
-    const float L = sum + wb;
-    if (t == 0) {
-      s_ml[0] = mx;
-      s_ml[1] = L == 0.f ? 0.f : 1.f / L;
-      if (p.lse_out) p.lse_out[qrow] = L == 0.f ? neg_inf() : mx + __logf(L);
-    }
-  }
-  __syncthreads();
-  if (merging) {
-    const float mx = s_ml[0];
-    const float inv = s_ml[1];
-    const float wb = (FMT >= 0 && mx != neg_inf()) ? __expf(lb - mx) : 0.f;
-    float4 a = wb > 0.f ? make_float4(wb * ob.x, wb * ob.y, wb * ob.z, wb * ob.w)
-                        : make_float4(0.f, 0.f, 0.f, 0.f);
-    if (pieces) {
-      if (n <= 8)
-        accum_preloaded(pv, n, s_w, a);
-      else
-        accum_pieces(pieces + 4 * c, sstride, n, s_w, a);
-    } else {
-      const float w = s_w[0];
-      a.x += w * v1.x; a.y += w * v1.y; a.z += w * v1.z; a.w += w * v1.w;
-    }
-    const float4 o = make_float4(a.x * inv, a.y * inv, a.z * inv, a.w * inv);
+  if (PS > 1) __syncthreads();
+  if (first == 0) {
+    float4 o;
+    float lse;
+    if constexpr (PS > 1)
+      merge_finish([&](int i) { return s_acc[i][c]; }, PS, lb, ob, o, lse);
+    else
+      merge_finish([&](int) { return x; }, 1, lb, ob, o, lse);
     uint2 packed;
     packed.x = pack_bf16x2(o.x, o.y);
     packed.y = pack_bf16x2(o.z, o.w);
-    if (p.out_bf16) ((uint2*)(p.out_bf16 + (size_t)qrow * p.Dv))[c] = packed;
+    if (p.out_bf16) ((uint2*)(p.out_bf16 + (size_t)qrow * Dv))[c] = packed;
+    if (p.lse_out && c == 0) p.lse_out[qrow] = lse;
     s_row[4 * c + 0] = bf16_to_f32(packed.x & 0xffffu);
     s_row[4 * c + 1] = bf16_to_f32(packed.x >> 16);
     s_row[4 * c + 2] = bf16_to_f32(packed.y & 0xffffu);
@@ -333,7 +373,7 @@ __global__ __launch_bounds__(kUvThreads) void merge_split_uv_kernel(
   }
   __syncthreads();
   // out_v[b][h * Dout + v] = sum_k s_row[k] * W_UV[h][v][k]: eight lanes per
-  // W_UV row, 32 rows per pass, kUvGroup passes per group of loads
+  // W_UV row, kUvThreads / 8 rows per pass, kUvGroup passes per group of loads
   for (int v0 = 0; v0 < Dout; v0 += kUvGroup * (kUvThreads / 8)) {
     if (v0 > 0) {  // groups after the first load here
 #pragma unroll
@@ -367,29 +407,39 @@ __global__ __launch_bounds__(kUvThreads) void merge_split_uv_kernel(
 }
 
 
-// Split combine without a host partial (the one-launch GQA entry points):
-// one 64-lane workgroup per output row, Dv <= 256 so a row is one column
-// chunk and out/lse may alias out_g/lse_g; out_bf16 (optional) receives the
-// same output rounded to bf16.
-int merge_split_pieces(const int32_t* len, int len_add, int B, int R, int heads, int Dv,
-                       int cap, int n, const float* out_g, const float* lse_g,
-                       const SplitWorkspace& w, float* out, float* lse, uint16_t* out_bf16,
-                       hipStream_t stream) {
-  if (Dv > 4 * kMergeChunk4)
-    return set_error(WS_EINVAL, "merge_split_pieces: Dv %d > %d", Dv, 4 * kMergeChunk4);
+// Launches merge_split_uv_kernel<FMT> (the plan rows are p.B: R = 1).
+template <int FMT>
+static void launch_merge_uv(const MergeSplitParams& p, const uint16_t* w_uv, int Dout,
+                            uint16_t* out_v, hipStream_t s) {
+  const dim3 grid((unsigned)(p.B / p.ng * p.heads)), block(kUvThreads);
+  const int PS = merge_streams(p.grid, p.B, merge_groups(p.heads / p.ng, p.Dv / 4));
+  if (PS == kMergeMaxStreams)
+    hipLaunchKernelGGL((merge_split_uv_kernel<FMT, kMergeMaxStreams>), grid, block, 0, s, p, w_uv,
+                       Dout, out_v);
+  else if (PS == 4)
+    hipLaunchKernelGGL((merge_split_uv_kernel<FMT, 4>), grid, block, 0, s, p, w_uv, Dout, out_v);
+  else
+    hipLaunchKernelGGL((merge_split_uv_kernel<FMT, 1>), grid, block, 0, s, p, w_uv, Dout, out_v);
+}
+
+// Split combine without a host partial (the one-launch entry points).
+int merge_split_pieces(const int32_t* len, int len_add, const MlaLayout& lay, int R, int heads,
+                       int Dv, int cap, int n, float* out, float* lse, const SplitWorkspace& w,
+                       uint16_t* out_bf16, hipStream_t stream) {
   MergeSplitParams prm;
   prm.gpu_len = len;
-  prm.B = B;
-  prm.ng = 1;
-  prm.step = kAlignStep;
+  prm.B = lay.plan_seqs;
+  prm.ng = lay.ng;
+  prm.step = lay.step;
+  prm.in_place = out_bf16 == nullptr;
   prm.R = R;
   prm.heads = heads;
   prm.Dv = Dv;
   prm.cap = cap;
   prm.grid = n;
   prm.add = len_add;
-  prm.out_g = out_g;
-  prm.lse_g = lse_g;
+  prm.out_g = out;
+  prm.lse_g = lse;
   prm.part_out = w.part_out;
   prm.part_lse = w.part_lse;
   prm.b_out = nullptr;
@@ -398,8 +448,7 @@ int merge_split_pieces(const int32_t* len, int len_add, int B, int R, int heads,
   prm.out_bf16 = out_bf16;
   prm.out_f32 = out;
   prm.lse_out = lse;
-  hipLaunchKernelGGL(merge_split_kernel<-1>, dim3((unsigned)(B * R * heads)), dim3(64),
-                     merge_lds(n), stream, prm);
+  launch_merge<-1>(prm, (long long)lay.plan_seqs * R, stream);
   return WS_OK;
 }
 
@@ -477,33 +526,17 @@ extern "C" int ws_merge_split(const int32_t* gpu_len, int B, int rows_per_seq, i
   prm.out_bf16 = out_bf16;
   prm.out_f32 = out_f32;
   prm.lse_out = lse_out;
-  const dim3 grid((unsigned)(rows_kv * heads), (unsigned)((Dv / 4 + kMergeChunk4 - 1) / kMergeChunk4));
-  const dim3 block(64);
+  prm.in_place = false;
   hipStream_t s = (hipStream_t)stream;
   if (!b_out) {
-    hipLaunchKernelGGL(merge_split_kernel<-1>, grid, block, merge_lds(n_workgroups), s, prm);
+    launch_merge<-1>(prm, rows_kv, s);
   } else {
     switch (fmt_b) {
-      case WS_PARTIAL_LSE_F32:
-        hipLaunchKernelGGL(merge_split_kernel<WS_PARTIAL_LSE_F32>, grid, block, merge_lds(n_workgroups),
-                           s, prm);
-        break;
-      case WS_TRIPLE_UNNORM_F32:
-        hipLaunchKernelGGL(merge_split_kernel<WS_TRIPLE_UNNORM_F32>, grid, block, merge_lds(n_workgroups),
-                           s, prm);
-        break;
-      case WS_TRIPLE_NORM_BF16:
-        hipLaunchKernelGGL(merge_split_kernel<WS_TRIPLE_NORM_BF16>, grid, block, merge_lds(n_workgroups),
-                           s, prm);
-        break;
-      case WS_PARTIAL_LSE_BF16:
-        hipLaunchKernelGGL(merge_split_kernel<WS_PARTIAL_LSE_BF16>, grid, block, merge_lds(n_workgroups),
-                           s, prm);
-        break;
-      default:
-        hipLaunchKernelGGL(merge_split_kernel<WS_TRIPLE_NORM_F32>, grid, block, merge_lds(n_workgroups),
-                           s, prm);
-        break;
+      case WS_PARTIAL_LSE_F32: launch_merge<WS_PARTIAL_LSE_F32>(prm, rows_kv, s); break;
+      case WS_TRIPLE_UNNORM_F32: launch_merge<WS_TRIPLE_UNNORM_F32>(prm, rows_kv, s); break;
+      case WS_TRIPLE_NORM_BF16: launch_merge<WS_TRIPLE_NORM_BF16>(prm, rows_kv, s); break;
+      case WS_PARTIAL_LSE_BF16: launch_merge<WS_PARTIAL_LSE_BF16>(prm, rows_kv, s); break;
+      default: launch_merge<WS_TRIPLE_NORM_F32>(prm, rows_kv, s); break;
     }
   }
   return check_launch("ws_merge_split");
@@ -603,34 +636,23 @@ extern "C" int ws_mla_merge_split_uv(const int32_t* gpu_len, int B, int heads,
   prm.out_bf16 = out_latent;
   prm.out_f32 = nullptr;
   prm.lse_out = lse_out;
-  const dim3 grid((unsigned)(B * heads));
-  const dim3 block(kUvThreads);
+  prm.in_place = false;
   hipStream_t s = (hipStream_t)stream;
   if (!b_out) {
-    hipLaunchKernelGGL(merge_split_uv_kernel<-1>, grid, block, merge_lds(n_workgroups), s, prm, w_uv,
-                       Dout, out_v);
+    launch_merge_uv<-1>(prm, w_uv, Dout, out_v, s);
   } else {
     switch (fmt_b) {
-      case WS_PARTIAL_LSE_F32:
-        hipLaunchKernelGGL(merge_split_uv_kernel<WS_PARTIAL_LSE_F32>, grid, block, merge_lds(n_workgroups), s,
-                           prm, w_uv, Dout, out_v);
-        break;
+      case WS_PARTIAL_LSE_F32: launch_merge_uv<WS_PARTIAL_LSE_F32>(prm, w_uv, Dout, out_v, s); break;
       case WS_TRIPLE_UNNORM_F32:
-        hipLaunchKernelGGL(merge_split_uv_kernel<WS_TRIPLE_UNNORM_F32>, grid, block, merge_lds(n_workgroups), s,
-                           prm, w_uv, Dout, out_v);
+        launch_merge_uv<WS_TRIPLE_UNNORM_F32>(prm, w_uv, Dout, out_v, s);
         break;
       case WS_TRIPLE_NORM_BF16:
-        hipLaunchKernelGGL(merge_split_uv_kernel<WS_TRIPLE_NORM_BF16>, grid, block, merge_lds(n_workgroups), s,
-                           prm, w_uv, Dout, out_v);
+        launch_merge_uv<WS_TRIPLE_NORM_BF16>(prm, w_uv, Dout, out_v, s);
         break;
       case WS_PARTIAL_LSE_BF16:
-        hipLaunchKernelGGL(merge_split_uv_kernel<WS_PARTIAL_LSE_BF16>, grid, block, merge_lds(n_workgroups), s,
-                           prm, w_uv, Dout, out_v);
+        launch_merge_uv<WS_PARTIAL_LSE_BF16>(prm, w_uv, Dout, out_v, s);
         break;
-      default:
-        hipLaunchKernelGGL(merge_split_uv_kernel<WS_TRIPLE_NORM_F32>, grid, block, merge_lds(n_workgroups), s,
-                           prm, w_uv, Dout, out_v);
-        break;
+      default: launch_merge_uv<WS_TRIPLE_NORM_F32>(prm, w_uv, Dout, out_v, s); break;
     }
   }
   return check_launch("ws_mla_merge_split_uv");

@@ -12,7 +12,7 @@
 // online softmax, and wave w accumulates output columns [128w, 128w + 128).
 // A sequence held by one workgroup is written final (fp32 out / lse);
 // otherwise each workgroup stores a bf16 piece (slot workgroup + sequence,
-// 16 KB) and a later launch combines them: mla_reduce_kernel for the
+// 16 KB) and a later launch combines them: merge_split_pieces for the
 // one-launch entry points, ws_merge_split / ws_mla_merge_split_uv for the
 // split step.
 //
@@ -55,7 +55,6 @@ struct MlaParams {
   // The wide kernel plans sequences (ng = 1) with rows of all H heads.
   int B, ng, page_size, max_pages, num_pages, cap;
   int hp;  // heads of a piece (and of a plan sequence's rows): 16, or all H (wide)
-  int step;  // the plan's alignment step
   float scale_log2;
 };
 
@@ -410,53 +409,6 @@ __global__ __launch_bounds__(256) void mla_decode_kernel(const MlaParams p) {
 
 namespace ws {
 
-// Combines the partials of sequences held by several workgroups: one 64-lane
-// workgroup per (head row, 256-column chunk).  Recomputes the decode's plan
-// to find the sequence's workgroups (slots w + b for w in its owner range).
-// Runs after the decode kernel on the same stream, so plain loads see the
-// partials.
-__global__ __launch_bounds__(64) void mla_reduce_kernel(const MlaParams p, int grid) {
-  extern __shared__ float s_w[];  // weights of the row's pieces (at most grid)
-  const int hrow = blockIdx.x;  // b * hp + h
-  const int chunk = blockIdx.y;
-  const int t = threadIdx.x;
-  const int b = hrow / p.hp;
-  const int h = hrow - b * p.hp;
-  const int add = p.c_new ? 1 : 0;
-  const RowSplits rs = plan_row(p.len_in, add, p.cap, p.B, 1, grid, b, 0, p.ng, p.step);
-  const int n = rs.nseg;
-  if (n <= 1) return;
-  const size_t slot0 = (size_t)(rs.w_first + b) * p.hp + h;  // partial row of split 0
-  const int c = chunk * 64 + t;  // float4 column
-  // the pieces' columns are requested with their lse values
-  uint2 pv[8];
-  if (n <= 8) preload_pieces(p.part_out + slot0 * kMlaC + 4 * c, (size_t)p.hp * kMlaC, n, pv);
-  float mx = neg_inf();
-  for (int s = t; s < n; s += 64) {
-    const float v = p.part_lse[slot0 + (size_t)s * p.hp];
-    s_w[s] = v;
-    mx = max_nan(mx, v);
-  }
-  for (int o = 1; o < 64; o <<= 1) mx = max_nan(mx, __shfl_xor(mx, o));
-  float sum = 0.f;
-  for (int s = t; s < n; s += 64) {
-    const float w = __expf(s_w[s] - mx);
-    s_w[s] = w;
-    sum += w;
-  }
-  for (int o = 1; o < 64; o <<= 1) sum += __shfl_xor(sum, o);
-  __syncthreads();
-  if (chunk == 0 && t == 0) p.lse[hrow] = mx + __logf(sum);
-  float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (n <= 8)
-    accum_preloaded(pv, n, s_w, a);
-  else
-    accum_pieces(p.part_out + slot0 * kMlaC + 4 * c, (size_t)p.hp * kMlaC, n, s_w, a);
-  const float inv = 1.f / sum;
-  ((float4*)(p.out + (size_t)hrow * kMlaC))[c] =
-      make_float4(a.x * inv, a.y * inv, a.z * inv, a.w * inv);
-}
-
 static bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 // Workgroups of an MLA call: n_workgroups when given, else one per CU (the
@@ -543,7 +495,6 @@ static int mla_launch(const uint16_t* q_nope, const uint16_t* q_pe,
   prm.B = Bv;
   prm.ng = ng;
   prm.hp = hp;
-  prm.step = lay.step;
   prm.page_size = page_size;
   prm.max_pages = max_pages;
   prm.num_pages = num_pages;
@@ -562,9 +513,9 @@ static int mla_launch(const uint16_t* q_nope, const uint16_t* q_pe,
   }
   int rc = check_launch(name);
   if (rc || n == 1 || !combine) return rc;
-  hipLaunchKernelGGL(mla_reduce_kernel, dim3(Bv * hp, kMlaC / 256), dim3(64),
-                     4 * (size_t)n, s, prm, n);
-  return check_launch(name);
+  rc = merge_split_pieces(len_in, c_new ? 1 : 0, lay, 1, hp, kMlaC, prm.cap, n, out, lse, w,
+                          nullptr, s);
+  return rc != WS_OK ? rc : check_launch(name);
 }
 
 }  // namespace ws

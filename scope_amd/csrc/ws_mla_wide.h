@@ -58,8 +58,7 @@
 //
 // Plan (ws_plan.h) over sequences; a sequence held by one workgroup is written
 // final (fp32 out / lse), otherwise each workgroup leaves a bf16 piece of all
-// its heads in slot workgroup + sequence, which mla_reduce_kernel or the merges
-// combine.  A workgroup that enters a second sequence pays a start and an end
+// its heads in slot workgroup + sequence, which the merges combine.  A workgroup that enters a second sequence pays a start and an end
 // again (about 14 us: ten blocks' time), so the plan prefers ranges of one
 // sequence (kAlignStepWide).  128 heads, B = 96 of 256 to 4096 tokens, step and
 // merge: 380 us as eight 16-head groups a sequence, 103 here; B = 40 of 500 to

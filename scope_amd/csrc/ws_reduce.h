@@ -5,8 +5,7 @@
 // normalised fp32, lse natural log) straight to the caller's out / lse; a
 // row spread over several splits leaves one piece per split in the
 // workspace, and a later launch on the same stream (merge_split_kernel,
-// merge_split_uv_kernel, mla_reduce_kernel) rebuilds the plan to find and
-// LSE-combine them.
+// merge_split_uv_kernel) rebuilds the plan to find and LSE-combine them.
 //
 // Workspace layout (ws_decode_plan), for a call over rows_kv rows of `heads`
 // output rows each, run by n splits:
@@ -92,14 +91,14 @@ int choose_workgroups(int n_workgroups, int per_cu, long long max_blocks, int mi
 // Workgroups of an MLA call (ws_mla.hip).
 int mla_workgroups(int n_workgroups, int B, int max_len);
 // Combines the pieces of a split decode step with no host partial: rows held
-// by several splits are LSE-combined from the workspace, the others copied;
-// lengths are len[b] + len_add; out/lse may alias out_g/lse_g (Dv <= 256);
-// out_bf16, when not null, also receives the output in bf16.  Launches on
-// `stream`; returns WS_OK or an error code (ws_merge.hip).
-int merge_split_pieces(const int32_t* len, int len_add, int B, int R, int heads, int Dv,
-                       int cap, int n, const float* out_g, const float* lse_g,
-                       const SplitWorkspace& w, float* out, float* lse, uint16_t* out_bf16,
-                       hipStream_t stream);
+// by several splits are LSE-combined from the workspace into out / lse, which
+// already hold the others; out_bf16, when not null, receives every row's output
+// in bf16.  lay gives the plan (B plan sequences of R rows; for absorbed MLA
+// the layout's); lengths are len[b] + len_add.  Launches on `stream`; returns
+// WS_OK or an error code (ws_merge.hip).
+int merge_split_pieces(const int32_t* len, int len_add, const MlaLayout& lay, int R, int heads,
+                       int Dv, int cap, int n, float* out, float* lse, const SplitWorkspace& w,
+                       uint16_t* out_bf16, hipStream_t stream);
 
 // Eight outputs of a piece, rounded to bf16, as one 16-byte store.
 __device__ __forceinline__ void store_piece8(uint16_t* dst, float a0, float a1, float a2,
@@ -121,60 +120,73 @@ __device__ __forceinline__ float4 piece4_f32(uint2 v) {
                      __builtin_bit_cast(float, v.y & 0xffff0000u));
 }
 
-// a += ws * (four outputs of one piece).
-__device__ __forceinline__ void accum_piece(float4& a, float ws, uint2 raw) {
-  const float4 v = piece4_f32(raw);
-  a.x += ws * v.x; a.y += ws * v.y; a.z += ws * v.z; a.w += ws * v.w;
+// Running LSE combine of part of a row's pieces in one thread's four columns:
+// sum and a are relative to m.
+struct PieceAcc {
+  float m, sum;
+  float4 a;
+};
+__device__ __forceinline__ PieceAcc piece_acc_empty() {
+  return PieceAcc{neg_inf(), 0.f, make_float4(0.f, 0.f, 0.f, 0.f)};
 }
 
-// a += sum_s w[s] * (four bf16 outputs of piece s at src + s * stride), in
-// order of s, with sixteen pieces' loads in flight per round while sixteen
-// remain, then eight (the last n % 8 pieces' loads also go out together).
-__device__ __forceinline__ void accum_pieces(const uint16_t* src, size_t stride, int n,
-                                             const float* w, float4& a) {
-  int s = 0;
-  for (; s + 16 <= n; s += 16) {
-    uint2 v[16];
+// exp(x - m): 0 for x = -inf (no weight) also where m is -inf, NaN for a NaN x.
+__device__ __forceinline__ float piece_weight(float x, float m) {
+  return x == neg_inf() ? 0.f : __expf(x - m);
+}
+// Factor that takes an accumulator from reference m to M >= m (an empty one, m
+// = -inf, holds only zeros, or the NaN of a bad piece, which stays).
+__device__ __forceinline__ float acc_factor(float m, float M) {
+  return m == neg_inf() ? 1.f : __expf(m - M);
+}
+
+// Adds the pieces s, s + step, ... (U of them, those below n) to an
+// accumulator: all U lse values and columns are requested before the first is
+// used (past n the last piece again, a cache hit).
+template <int U>
+__device__ __forceinline__ void piece_batch(PieceAcc& x, const uint16_t* pieces, size_t stride,
+                                            const float* lse, int lstride, int s, int step,
+                                            int n) {
+  float l[U];
+  uint2 v[U];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) v[u] = *(const uint2*)(src + (size_t)(s + u) * stride);
+  for (int u = 0; u < U; ++u) l[u] = lse[(size_t)min(s + u * step, n - 1) * lstride];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) accum_piece(a, w[s + u], v[u]);
+  for (int u = 0; u < U; ++u)
+    v[u] = *(const uint2*)(pieces + (size_t)min(s + u * step, n - 1) * stride);
+  float m = x.m;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (s + u * step >= n) l[u] = neg_inf();
+    m = fmaxf(m, l[u]);
   }
-  for (; s + 8 <= n; s += 8) {
-    uint2 v[8];
+  const float f = acc_factor(x.m, m);
+  x.m = m;
+  x.sum *= f;
+  x.a.x *= f; x.a.y *= f; x.a.z *= f; x.a.w *= f;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = *(const uint2*)(src + (size_t)(s + u) * stride);
-#pragma unroll
-    for (int u = 0; u < 8; ++u) accum_piece(a, w[s + u], v[u]);
-  }
-  if (s < n) {
-    uint2 v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-      v[u] = *(const uint2*)(src + (size_t)min(s + u, n - 1) * stride);
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-      if (s + u < n) accum_piece(a, w[s + u], v[u]);
+  for (int u = 0; u < U; ++u) {
+    if (s + u * step >= n) continue;
+    const float w = piece_weight(l[u], m);
+    const float4 o = piece4_f32(v[u]);
+    x.sum += w;
+    x.a.x += w * o.x; x.a.y += w * o.y; x.a.z += w * o.z; x.a.w += w * o.w;
   }
 }
 
-// The raw bytes of a row's pieces when it has at most eight (a row with
-// fewer repeats its last one), requested before the weights are known: the
-// piece loads share their round trip with the lse loads, and nothing waits
-// for them until the accumulation.
-__device__ __forceinline__ void preload_pieces(const uint16_t* src, size_t stride, int n,
-                                               uint2 (&v)[8]) {
-#pragma unroll
-  for (int u = 0; u < 8; ++u) v[u] = *(const uint2*)(src + (size_t)min(u, n - 1) * stride);
-}
-
-// accum_pieces over the n <= 8 pieces preload_pieces fetched: the same terms
-// in the same order, so the result is bit-identical to accum_pieces.
-__device__ __forceinline__ void accum_preloaded(const uint2 (&v)[8], int n, const float* w,
-                                                float4& a) {
-#pragma unroll
-  for (int u = 0; u < 8; ++u)
-    if (u < n) accum_piece(a, w[u], v[u]);
+// The pieces first, first + step, ... of a row's n.
+__device__ __forceinline__ PieceAcc piece_stream(const uint16_t* pieces, size_t stride,
+                                                 const float* lse, int lstride, int first,
+                                                 int step, int n) {
+  PieceAcc x = piece_acc_empty();
+  int s = first;
+  for (; s + 8 * step < n; s += 16 * step)
+    piece_batch<16>(x, pieces, stride, lse, lstride, s, step, n);
+  if (s + 4 * step < n)
+    piece_batch<8>(x, pieces, stride, lse, lstride, s, step, n);
+  else if (s < n)
+    piece_batch<4>(x, pieces, stride, lse, lstride, s, step, n);
+  return x;
 }
 
 }  // namespace ws
