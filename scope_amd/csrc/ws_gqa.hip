@@ -44,11 +44,6 @@ constexpr int kGqaWaves = 2;        // waves per workgroup, each its own split
 constexpr int kGqaStages = 2;       // register stages of a wave's load ring
 constexpr int kGqaSplitsPerCu = 2;  // default splits (waves) per CU
 
-// Register stages of the ring: two 256-wide K and V stages (256 VGPRs) do
-// not fit beside the accumulators and q even in the 512 registers of one wave
-// per SIMD (the compiler spilled 730 bytes per lane), so 256-wide values
-// stream one block per wave at a time.
-__host__ __device__ constexpr int gqa_stages(int DV) { return DV > kGqaD ? 1 : kGqaStages; }
 // Waves per SIMD the kernel is compiled for (its register budget): rings
 // wider than 128 need the 512 registers of one wave per SIMD, and so does the
 // 128-wide ring with the group size read at run time (G = 0: it spilled in
@@ -67,6 +62,21 @@ __host__ __device__ constexpr int gqa_lane_cols(int DV) {
   while (DV % c) c += 2;
   return c;
 }
+
+// Register stages of the K and V rings.  Two 256-wide K and V stages (256
+// VGPRs) do not fit beside the accumulators and q even in the 512 registers of
+// one wave per SIMD (the compiler spilled 730 bytes per lane, and 620 with two
+// K stages and one V stage: 190 us where one of each takes 60).  Values wider
+// than 128 of at most 12 columns (accumulator tiles) a lane, 144, 160 and 192,
+// keep two K stages and one V stage, which is requested as soon as the block
+// before has used it and arrives under the next block's scores; the others
+// stream one block per wave at a time.  (One stage of each for these too, 8
+// sequences of 1000 to 16384 tokens, 4 x 2 heads, us a step: D = 144 50.4, 160
+// 42.1, 192 49.7; now 39.7, 38.7, 43.4.)
+__host__ __device__ constexpr int gqa_k_stages(int DV) {
+  return gqa_lane_cols(DV) > 12 ? 1 : kGqaStages;
+}
+__host__ __device__ constexpr int gqa_v_stages(int DV) { return DV > kGqaD ? 1 : kGqaStages; }
 
 // N dwords of a lane's V columns: 8, 16 or 32 bytes as vector loads, other
 // sizes as dword arrays (4, 12, 20, 24 or 28 bytes: 4-byte aligned only).
@@ -234,10 +244,9 @@ gqa_decode_kernel(
   // k_new/v_new.  With valid == false (the request past the range's last
   // block) every lane reads the first row of q instead: same instructions
   // and registers, a cache hit, no HBM traffic.
-  auto load_block = [&](const GqaBlock& m, bool valid, u32x4 (&ka)[2][KS],
-                        VT (&vr)[8]) __attribute__((always_inline)) {
+  auto load_k = [&](const GqaBlock& m, bool valid,
+                    u32x4 (&ka)[2][KS]) __attribute__((always_inline)) {
     const uint16_t* kb = valid ? p.k_pages + (size_t)m.tok * DK : p.q;
-    const uint16_t* vb = valid ? p.v_pages + (size_t)m.tok * D : p.q;
     const int last = valid ? (m.nt & kNtMask) - 1 : 0;
     const int new_r = (APPEND && valid) ? m.nr : -1;
 #pragma unroll
@@ -248,6 +257,11 @@ gqa_decode_kernel(
 #pragma unroll
       for (int s = 0; s < KS; ++s) ka[tt][s] = ld_stream(kr + kcol(s, j));
     }
+  };
+  auto load_v = [&](const GqaBlock& m, bool valid, VT (&vr)[8]) __attribute__((always_inline)) {
+    const uint16_t* vb = valid ? p.v_pages + (size_t)m.tok * D : p.q;
+    const int last = valid ? (m.nt & kNtMask) - 1 : 0;
+    const int new_r = (APPEND && valid) ? m.nr : -1;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int r = min(pv_token(i, j), last);
@@ -392,21 +406,25 @@ gqa_decode_kernel(
   // Ring of S register stages: stage st holds the block k with k % S == st
   // and its metadata mq[st].  Step k requests block k + S - 1 into stage
   // (k + S - 1) % S, then runs block k's math; past the range's end the
-  // request is the q-row dummy of load_block.  After block k's math, qb
+  // request is the q-row dummy of the loads.  After block k's math, qb
   // takes the q rows of block k + 1's kv row (an L2 hit, issued every block
   // so that no load in the loop is conditional), ahead of the next block
-  // requests, so waiting for it costs nothing extra.  sched_barrier keeps
+  // requests, so waiting for it costs nothing extra.  A single V stage (SV)
+  // beside two K stages takes block k + 1's V after block k's math, behind q:
+  // the next scores then wait for K and q, and not for V.  sched_barrier keeps
   // the compiler from sinking the loads below the math (which would
   // serialise them again).  The loop body is a whole turn of the ring with no
   // early exit (the last nblk % S blocks run after it): a path around one
   // step would make the compiler assume that step's loads are still in
   // flight when the ring comes back to it, and wait.
-  constexpr int S = gqa_stages(DV);
+  constexpr int S = gqa_k_stages(DV);
+  constexpr int SV = gqa_v_stages(DV);
+  static_assert(S <= 2 && SV <= S, "a single V stage is free when block k + 1 is next");
   int xb = x_begin;
   fetch_meta(xb);
   GqaBlock mq[S];
   u32x4 ka[S][2][KS];
-  VT vr[S][8];
+  VT vr[SV][8];
   mq[0] = read_meta(0);
   int run_row = mq[0].row;
   bool run_first = (mq[0].nt & kFirst) != 0;  // the running row's first block was ours
@@ -417,7 +435,8 @@ gqa_decode_kernel(
     constexpr int st = decltype(i)::value;
     const bool valid = st < nblk;
     if (st > 0) mq[st] = valid ? read_meta(st) : mq[0];
-    load_block(mq[st], valid, ka[st], vr[st]);
+    load_k(mq[st], valid, ka[st]);
+    load_v(mq[st], valid, vr[st % SV]);
   });
   auto step = [&](auto stage, int k) __attribute__((always_inline)) {
     constexpr int st = decltype(stage)::value;
@@ -430,7 +449,8 @@ gqa_decode_kernel(
     }
     if (S > 1) mq[ld] = valid ? read_meta(x_begin + k + S - 1 - xb) : mq[st];
     else mq[0] = read_meta(x_begin + k - xb);  // (one stage: block k itself, always valid)
-    load_block(mq[ld], valid, ka[ld], vr[ld]);
+    load_k(mq[ld], valid, ka[ld]);
+    if (SV == S) load_v(mq[ld], valid, vr[ld % SV]);
     if (S == 1) load_q(mq[0].row);
     __builtin_amdgcn_sched_barrier(0);
     const GqaBlock& cur = mq[st];
@@ -446,11 +466,15 @@ gqa_decode_kernel(
     }
     run_last = (cur.nt & kLast) != 0;
     run_bad |= (cur.nt & kBadPage) != 0;
-    compute_block(cur, ka[st], vr[st]);
+    compute_block(cur, ka[st], vr[st % SV]);
     __builtin_amdgcn_sched_barrier(0);
     // (One stage: block k + 1's row is not known yet; its step requests q
     // right after its block.)
     if (S > 1) load_q(mq[nx].row);
+    if (SV < S) {
+      __builtin_amdgcn_sched_barrier(0);
+      load_v(mq[ld], valid, vr[0]);
+    }
   };
   int base = 0;
   for (; base + S <= nblk; base += S)
