@@ -154,18 +154,25 @@ def _check(rc: int, name: str) -> None:
         raise WsError(f"{name}: {lib().ws_last_error().decode()} (rc={rc})")
 
 
+# Addresses go to the library as plain integers: the argtypes convert them, and
+# a c_void_p object per argument cost 0.2 us each.
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _stream(device: torch.device):
     """The current HIP stream of `device` (the raw handle torch launches on)."""
     idx = device.index if device.index is not None else torch.cuda.current_device()
-    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(idx))
+    return torch._C._cuda_getCurrentRawStream(idx)
 
 
 def _require(t: torch.Tensor, name: str, dtype: torch.dtype, device=None,
              ndim=None, contiguous=True) -> None:
+    if (isinstance(t, torch.Tensor) and t.dtype is dtype and t.is_cuda
+            and (device is None or t.device == device) and (ndim is None or t.dim() == ndim)
+            and (not contiguous or t.is_contiguous())):
+        return
+    # what is wrong, in this order
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a tensor")
     if not t.is_cuda:
@@ -215,7 +222,7 @@ def decode_plan(kind: int, rows_kv: int, heads: int, max_len: int,
     # the answer depends on the arguments and the current device only (a
     # decode loop asks the same question for every layer of a step)
     key = (kind, rows_kv, heads, max_len, n_workgroups,
-           torch.cuda.current_device() if torch.cuda.is_initialized() else -1)
+           torch._C._cuda_getDevice() if torch.cuda.is_initialized() else -1)
     hit = _plans.get(key)
     if hit is not None:
         return hit
@@ -235,7 +242,7 @@ def gqa_plan(rows_kv: int, heads: int, Dk: int, Dv: int, max_len: int,
     if Dk == 128 and Dv == 128:
         return decode_plan(0, rows_kv, heads, max_len, n_workgroups)
     key = ("attn", rows_kv, heads, Dk, Dv, max_len, n_workgroups,
-           torch.cuda.current_device() if torch.cuda.is_initialized() else -1)
+           torch._C._cuda_getDevice() if torch.cuda.is_initialized() else -1)
     hit = _plans.get(key)
     if hit is not None:
         return hit
