@@ -138,6 +138,14 @@ int ws_latent_append(const uint16_t* c_new, int64_t c_stride,
                      int num_pages, int update_len, void* stream);
 
 /*
+ * Paging of n contiguous per-row buffers (page_size = the rows' capacity,
+ * max_pages = 1): page_table[i] = i, gpu_len[i] = tokens, and ones[0..n_ones) =
+ * 1 (NULL with n_ones = 0 for none), in one launch.
+ */
+int ws_dense_paging(int32_t* page_table, int32_t* gpu_len, int n, int tokens, float* ones,
+                    int64_t n_ones, void* stream);
+
+/*
  * Plan of a decode call: kind 0 (GQA: rows_kv = B * Hkv, heads = the group
  * size G) or 1 (MLA: rows_kv = B, heads = H, a multiple of 16; H = 128, and
  * 32 <= H < 128 from B * H = 1024, plan sequences with H-head pieces, others

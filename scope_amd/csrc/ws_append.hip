@@ -35,6 +35,21 @@ __device__ __forceinline__ bool append_ok(const int32_t* __restrict__ pt_row, in
   return !__syncthreads_or(bad);
 }
 
+// Paging of contiguous per-row buffers (row n is page n) and the ones of their
+// partial's triple, in one launch: a fill each made three launches, 3.7 us of a
+// step of 65.7 over 128 rows of 4k tokens (192 / 128 wide).
+__global__ __launch_bounds__(256) void dense_paging_kernel(int32_t* __restrict__ page_table,
+                                                           int32_t* __restrict__ len, int n,
+                                                           int tokens, float* __restrict__ ones,
+                                                           long long n_ones) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) {
+    page_table[i] = (int32_t)i;
+    len[i] = tokens;
+  }
+  if (i < n_ones) ones[i] = 1.f;
+}
+
 // Length update of a multi-chunk append: one workgroup per sequence.
 __global__ __launch_bounds__(256) void len_add_kernel(int32_t* __restrict__ gpu_len,
                                                       const int32_t* __restrict__ page_table,
@@ -192,4 +207,18 @@ extern "C" int ws_latent_append(const uint16_t* c_new, int64_t c_stride,
     hipLaunchKernelGGL(len_add_kernel, dim3(B), dim3(256), 0, s, gpu_len, page_table, n_new,
                        page_size, max_pages, num_pages);
   return check_launch("ws_latent_append");
+}
+
+extern "C" int ws_dense_paging(int32_t* page_table, int32_t* gpu_len, int n, int tokens,
+                               float* ones, int64_t n_ones, void* stream) {
+  if ((n > 0 && (!page_table || !gpu_len)) || (n_ones > 0 && !ones))
+    return set_error(WS_EINVAL, "ws_dense_paging: null pointer");
+  if (n < 0 || tokens < 0 || n_ones < 0 || n_ones > (1LL << 31))
+    return set_error(WS_EINVAL, "ws_dense_paging: bad sizes n=%d tokens=%d n_ones=%lld", n, tokens,
+                     (long long)n_ones);
+  const long long most = n > n_ones ? n : n_ones;
+  if (most == 0) return WS_OK;
+  hipLaunchKernelGGL(dense_paging_kernel, dim3((unsigned)((most + 255) / 256)), dim3(256), 0,
+                     (hipStream_t)stream, page_table, gpu_len, n, tokens, ones, n_ones);
+  return check_launch("ws_dense_paging");
 }

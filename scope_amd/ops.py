@@ -28,6 +28,7 @@ EXPORTS = (
     "ws_version",
     "ws_kv_append",
     "ws_latent_append",
+    "ws_dense_paging",
     "ws_decode_plan",
     "ws_attn_decode_plan",
     "ws_gqa_decode_partial",
@@ -90,6 +91,8 @@ def lib() -> ctypes.CDLL:
         L.ws_latent_append.restype = i32
         L.ws_latent_append.argtypes = [vp, i64, vp, i64, vp, vp, vp, i32, i32,
                                        i32, i32, i32, i32, vp]
+        L.ws_dense_paging.restype = i32
+        L.ws_dense_paging.argtypes = [vp, vp, i32, i32, vp, i64, vp]
         L.ws_decode_plan.restype = i32
         L.ws_decode_plan.argtypes = [i32, i32, i32, i32, i32,
                                      ctypes.POINTER(i32), ctypes.POINTER(sz)]
@@ -210,6 +213,19 @@ def _workspace(device: torch.device, nbytes: int) -> torch.Tensor:
 
 
 _plans: dict = {}
+
+
+def dense_paging(n: int, tokens: int, ones_shape, device):
+    """(page_table [n, 1], lengths [n], ones) of n contiguous per-row buffers
+    that hold `tokens` tokens each (ws_dense_paging)."""
+    ints = torch.empty((2, n), dtype=torch.int32, device=device)
+    ones = torch.empty(ones_shape, dtype=torch.float32, device=device)
+    if not ints.is_cuda:
+        raise ValueError(f"device must be a GPU (got {device})")
+    _check(lib().ws_dense_paging(ints.data_ptr(), ints.data_ptr() + 4 * n, n, tokens,
+                                 _ptr(ones), ones.numel(), _stream(ints.device)),
+           "ws_dense_paging")
+    return ints[0].view(n, 1), ints[1], ones
 
 
 def decode_plan(kind: int, rows_kv: int, heads: int, max_len: int,

@@ -17,12 +17,6 @@ import torch
 from . import ops
 
 
-def _dense_paging(n: int, s: int, device):
-    page_table = torch.arange(n, dtype=torch.int32, device=device).view(n, 1)
-    gpu_len = torch.full((n,), s, dtype=torch.int32, device=device)
-    return page_table, gpu_len
-
-
 def local_bmm_softmax(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float,
                       n_workgroups: int = 0):
     """_local_bmm_softmax (roofline/bench_resident_kv.py:150-157).
@@ -40,11 +34,11 @@ def local_bmm_softmax(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: 
         return (torch.zeros((N, G, Dv), dtype=torch.float32, device=q.device),
                 torch.full((N, G, 1), float("-inf"), dtype=torch.float32, device=q.device),
                 torch.zeros((N, G, 1), dtype=torch.float32, device=q.device))
-    pt, ln = _dense_paging(N, S, q.device)
+    pt, ln, ones = ops.dense_paging(N, S, (N, G, 1), q.device)
     out, lse = ops.attn_decode_partial(q.contiguous(), k.contiguous().view(N, 1, S, Dk),
                                        v.contiguous().view(N, 1, S, Dv), pt, ln, scale, S,
                                        n_workgroups)
-    return out, lse.unsqueeze(-1), torch.ones_like(lse).unsqueeze(-1)
+    return out, lse.unsqueeze(-1), ones
 
 
 def pairwise_merge(o1, m1, s1, o2, m2, s2):
@@ -75,9 +69,9 @@ def resident_layer(q, k_buf, v_buf, new_k, new_v, scale):
                 torch.full((max(N, 0), G, 1), float("-inf"), dtype=torch.float32,
                            device=q.device),
                 torch.zeros((max(N, 0), G, 1), dtype=torch.float32, device=q.device))
-    pt, ln = _dense_paging(N, cap - 1, q.device)
+    pt, ln, ones = ops.dense_paging(N, cap - 1, (N, q.shape[1], 1), q.device)
     out, lse = ops.attn_decode_partial(
         q.contiguous(), k_buf.view(N, 1, cap, Dk), v_buf.view(N, 1, cap, Dv), pt, ln, scale,
         cap, k_new=new_k.contiguous().view(N, 1, 1, Dk),
         v_new=new_v.contiguous().view(N, 1, 1, Dv))
-    return out, lse.unsqueeze(-1), torch.ones_like(lse).unsqueeze(-1)
+    return out, lse.unsqueeze(-1), ones

@@ -148,3 +148,13 @@ def test_mla_many_sequences(B, H, wg):
         assert_close(mo[b], o, OUT_ATOL, OUT_RTOL, f"merged out {b}")
         assert_close(ml[b], l, LSE_ATOL, LSE_RTOL, f"merged lse {b}")
         assert_close(ov[b], torch.einsum("hk,hvk->hv", o, w), OUT_ATOL, OUT_RTOL, f"out_v {b}")
+
+
+@pytest.mark.parametrize("n,tokens,shape", [(1, 0, (1, 1, 1)), (3, 5, (3, 100, 1)),
+                                            (256, 4097, (256, 1, 1)), (2049, 7, (2049, 1, 1)),
+                                            (0, 3, (0, 4, 1))])
+def test_dense_paging(n, tokens, shape):
+    table, lens, ones = ops.dense_paging(n, tokens, shape, torch.device(DEV))
+    assert table.shape == (n, 1) and table.view(-1).tolist() == list(range(n))
+    assert lens.tolist() == [tokens] * n
+    assert ones.shape == shape and bool((ones == 1).all())
