@@ -310,8 +310,9 @@ int ws_attn_append_decode_partial(const uint16_t* q, const uint16_t* k_new,
  * DeepSeek-V2-Lite, 128 for DeepSeek-V2; nH = q rows / B as in
  * kernel/cpu_attn.cpp:860).  H = 128, and 32 <= H < 128 from B * H = 1024,
  * run one pass over each latent block for all heads (a workgroup of four
- * 32-head waves, pieces of H heads); other calls plan each group of 16 heads
- * as a sequence of its own over the shared latent.  A sequence's new latent is written once.
+ * 32-head waves, pieces of H heads, in fp32 except for 128 heads over at most
+ * 64 sequences); other calls plan each group of 16 heads as a sequence of its
+ * own over the shared latent.  A sequence's new latent is written once.
  * Outputs out: [B*H][512] fp32 normalised, lse: [B*H] fp32.
  * Replaces the GPU partial of _mla_compressed_forward
  * (system/deepseek.py:364-392; also roofline/bench_rstar_revalidate_ds2.py:74-86).

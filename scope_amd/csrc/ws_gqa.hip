@@ -647,7 +647,7 @@ static int gqa_launch(const uint16_t* q, const uint16_t* k_new, const uint16_t* 
   if (rc != WS_OK || !combine) return rc;
   // One-launch entry points: the rows held by several waves are combined by
   // the split merge on the same stream.
-  const MlaLayout lay = {false, 1, G, B, kAlignStep};
+  const MlaLayout lay = {false, 1, G, B, kAlignStep, false};
   rc = merge_split_pieces(len_in, k_new ? 1 : 0, lay, Hkv, G, D, prm.cap, n, out, lse, prm.ws,
                           out_bf16, s);
   return rc != WS_OK ? rc : check_launch(name);
@@ -667,7 +667,7 @@ extern "C" int ws_decode_plan(int kind, int rows_kv, int heads, int max_len,
   } else {  // one plan sequence per (sequence, 16-head group), or per sequence (wide)
     const MlaLayout lay = mla_layout(rows_kv, heads);
     n = mla_workgroups(n_workgroups, lay.plan_seqs, max_len);
-    bytes = ws::workspace_bytes(lay.plan_seqs, lay.piece_heads, 512, n);
+    bytes = ws::workspace_bytes(lay.plan_seqs, lay.piece_heads, 512, n, lay.f32_pieces);
   }
   if (n_workgroups_out) *n_workgroups_out = n;
   if (workspace_bytes_out) *workspace_bytes_out = bytes;

@@ -115,11 +115,12 @@ struct MergeSplitParams {
   // plan sequences are (sequence, 16-head group) pairs (ws_plan.h seq_of).
   int B, ng, R, heads, Dv, cap, grid;
   int step;       // the plan's alignment step
+  bool f32_pieces;
   bool in_place;  // out_g / lse_g are the outputs: rows of one piece stay as they are
   int add;  // lengths are gpu_len[b] + add (1 when gpu_len is a fused step's len_in)
   const float* out_g;
   const float* lse_g;
-  const uint16_t* part_out;  // bf16 pieces
+  const uint16_t* part_out;  // bf16 pieces (fp32 ones with f32_pieces)
   const float* part_lse;
   const void* b_out;
   const void* b_aux0;
@@ -173,15 +174,18 @@ __host__ __device__ inline int merge_groups(int heads, int Dv4) {
   return Dv4 <= 64 ? (heads + 64 / Dv4 - 1) / (64 / Dv4) : heads * ((Dv4 + 63) >> 6);
 }
 
-// What stream `st` of PS adds to the row's output: its share of the pieces, or
-// (the first stream) the final partial of a row that one split held.
+// What stream `st` of PS adds to the row's output: its share of the pieces (VT:
+// four columns of one, bf16 or fp32), or (the first stream) the final partial of
+// a row that one split held.
+template <class VT>
 __device__ __forceinline__ PieceAcc merge_stream(const MergeSplitParams& p, const RowSplits& rs,
                                                  size_t krow, int h, int c, int heads, int st,
                                                  int PS) {
   if (rs.nseg > 1) {
     const size_t slot0 = ((size_t)rs.w_first + krow) * heads + h;
-    return piece_stream(p.part_out + slot0 * p.Dv + 4 * c, (size_t)heads * p.Dv,
-                        p.part_lse + slot0, heads, st, PS, rs.nseg);
+    const size_t row = (size_t)(p.Dv >> 2) * sizeof(VT);  // bytes of a piece's row
+    return piece_stream<VT>((const char*)p.part_out + slot0 * row + c * sizeof(VT), heads * row,
+                            p.part_lse + slot0, heads, st, PS, rs.nseg);
   }
   PieceAcc x = piece_acc_empty();
   if (st == 0) {
@@ -219,7 +223,7 @@ __device__ __forceinline__ void merge_finish(const F& acc, int n, float lb, cons
   lse = L == 0.f ? neg_inf() : M + __logf(L);
 }
 
-template <int FMT, int PS>
+template <int FMT, int PS, class VT>
 __global__ __launch_bounds__(64 * (PS > kMergeWgWaves ? PS : kMergeWgWaves)) void
 merge_split_kernel(const MergeSplitParams p) {
   __shared__ PieceAcc s_acc[PS > 1 ? PS : 1][64];
@@ -258,14 +262,14 @@ merge_split_kernel(const MergeSplitParams p) {
   float4 o;
   float lse;
   if constexpr (PS > 1) {
-    s_acc[wave][lane] = merge_stream(p, rs, krow, mc.h, mc.c, p.heads, wave, PS);
+    s_acc[wave][lane] = merge_stream<VT>(p, rs, krow, mc.h, mc.c, p.heads, wave, PS);
     __syncthreads();
     if (wave != 0) return;
     merge_finish([&](int i) { return s_acc[i][lane]; }, PS, lb, ob, o, lse);
     store(o, lse);
   } else {
     for (;;) {
-      const PieceAcc x = merge_stream(p, rs, krow, mc.h, mc.c, p.heads, 0, 1);
+      const PieceAcc x = merge_stream<VT>(p, rs, krow, mc.h, mc.c, p.heads, 0, 1);
       merge_finish([&](int) { return x; }, 1, lb, ob, o, lse);
       store(o, lse);
       grp += waves * gridDim.y;
@@ -276,23 +280,28 @@ merge_split_kernel(const MergeSplitParams p) {
   }
 }
 
-// Launches merge_split_kernel<FMT> over rows plan rows.
+// Launches merge_split_kernel<FMT> over rows plan rows.  (fp32 pieces come with
+// at least 1024 output rows of 512 columns, mla_layout: 2048 column groups, so
+// one wave each.)
 template <int FMT>
 static void launch_merge(const MergeSplitParams& p, long long rows, hipStream_t s) {
   const int groups = merge_groups(p.heads, p.Dv / 4);
   const int PS = merge_streams(p.grid, rows, groups);
   if (PS == kMergeMaxStreams) {
-    hipLaunchKernelGGL((merge_split_kernel<FMT, kMergeMaxStreams>),
+    hipLaunchKernelGGL((merge_split_kernel<FMT, kMergeMaxStreams, uint2>),
                        dim3((unsigned)rows, groups), dim3(64 * kMergeMaxStreams), 0, s, p);
   } else if (PS == 4) {
-    hipLaunchKernelGGL((merge_split_kernel<FMT, 4>), dim3((unsigned)rows, groups), dim3(256), 0, s,
-                       p);
+    hipLaunchKernelGGL((merge_split_kernel<FMT, 4, uint2>), dim3((unsigned)rows, groups), dim3(256),
+                       0, s, p);
   } else {
     const int waves = std::min(groups, kMergeWgWaves);
     const long long fit = std::max(kMergeWaves / (rows * waves), 1LL);
     const int wgs = (int)std::min<long long>((groups + waves - 1) / waves, fit);
-    hipLaunchKernelGGL((merge_split_kernel<FMT, 1>), dim3((unsigned)rows, wgs), dim3(64 * waves), 0,
-                       s, p);
+    const dim3 grid((unsigned)rows, wgs), block(64 * waves);
+    if (p.f32_pieces)
+      hipLaunchKernelGGL((merge_split_kernel<FMT, 1, float4>), grid, block, 0, s, p);
+    else
+      hipLaunchKernelGGL((merge_split_kernel<FMT, 1, uint2>), grid, block, 0, s, p);
   }
 }
 
@@ -311,7 +320,7 @@ static void launch_merge(const MergeSplitParams& p, long long rows, hipStream_t 
 constexpr int kUvThreads = 256;
 constexpr int kUvGroup = 2;  // passes of 32 W_UV rows whose loads are in flight together
 
-template <int FMT, int PS>
+template <int FMT, int PS, class VT>
 __global__ __launch_bounds__(kUvThreads) void merge_split_uv_kernel(
     const MergeSplitParams p, const uint16_t* __restrict__ w_uv, int Dout,
     uint16_t* __restrict__ out_v) {
@@ -350,7 +359,7 @@ __global__ __launch_bounds__(kUvThreads) void merge_split_uv_kernel(
 #pragma unroll
   for (int i = 0; i < PS; i += kGroupWaves)
     if (first + i < PS) {
-      x = merge_stream(p, rs, pv_seq, h16, c, hp, first + i, PS);
+      x = merge_stream<VT>(p, rs, pv_seq, h16, c, hp, first + i, PS);
       if (PS > 1) s_acc[first + i][c] = x;
     }
   if (PS > 1) __syncthreads();
@@ -414,12 +423,17 @@ static void launch_merge_uv(const MergeSplitParams& p, const uint16_t* w_uv, int
   const dim3 grid((unsigned)(p.B / p.ng * p.heads)), block(kUvThreads);
   const int PS = merge_streams(p.grid, p.B, merge_groups(p.heads / p.ng, p.Dv / 4));
   if (PS == kMergeMaxStreams)
-    hipLaunchKernelGGL((merge_split_uv_kernel<FMT, kMergeMaxStreams>), grid, block, 0, s, p, w_uv,
-                       Dout, out_v);
+    hipLaunchKernelGGL((merge_split_uv_kernel<FMT, kMergeMaxStreams, uint2>), grid, block, 0, s, p,
+                       w_uv, Dout, out_v);
   else if (PS == 4)
-    hipLaunchKernelGGL((merge_split_uv_kernel<FMT, 4>), grid, block, 0, s, p, w_uv, Dout, out_v);
+    hipLaunchKernelGGL((merge_split_uv_kernel<FMT, 4, uint2>), grid, block, 0, s, p, w_uv, Dout,
+                       out_v);
+  else if (p.f32_pieces)
+    hipLaunchKernelGGL((merge_split_uv_kernel<FMT, 1, float4>), grid, block, 0, s, p, w_uv, Dout,
+                       out_v);
   else
-    hipLaunchKernelGGL((merge_split_uv_kernel<FMT, 1>), grid, block, 0, s, p, w_uv, Dout, out_v);
+    hipLaunchKernelGGL((merge_split_uv_kernel<FMT, 1, uint2>), grid, block, 0, s, p, w_uv, Dout,
+                       out_v);
 }
 
 // Split combine without a host partial (the one-launch entry points).
@@ -431,6 +445,7 @@ int merge_split_pieces(const int32_t* len, int len_add, const MlaLayout& lay, in
   prm.B = lay.plan_seqs;
   prm.ng = lay.ng;
   prm.step = lay.step;
+  prm.f32_pieces = lay.f32_pieces;
   prm.in_place = out_bf16 == nullptr;
   prm.R = R;
   prm.heads = heads;
@@ -499,7 +514,8 @@ extern "C" int ws_merge_split(const int32_t* gpu_len, int B, int rows_per_seq, i
   const long long rows_kv = (long long)Bp * rows_per_seq;
   if (rows_kv > (1 << 24))
     return set_error(WS_EINVAL, "ws_merge_split: %lld rows exceed %d", rows_kv, 1 << 24);
-  const size_t need = ws::workspace_bytes((int)rows_kv, heads, Dv, n_workgroups);
+  const bool f32_pieces = mla && lay.f32_pieces;
+  const size_t need = ws::workspace_bytes((int)rows_kv, heads, Dv, n_workgroups, f32_pieces);
   if (workspace_bytes < need)
     return set_error(WS_EWORKSPACE, "ws_merge_split: workspace %zu < %zu bytes",
                      workspace_bytes, need);
@@ -513,6 +529,7 @@ extern "C" int ws_merge_split(const int32_t* gpu_len, int B, int rows_per_seq, i
   prm.heads = heads;
   prm.Dv = Dv;
   prm.step = mla ? lay.step : kAlignStep;
+  prm.f32_pieces = f32_pieces;
   prm.cap = page_capacity;
   prm.grid = n_workgroups;
   prm.add = 0;
@@ -608,7 +625,8 @@ extern "C" int ws_mla_merge_split_uv(const int32_t* gpu_len, int B, int heads,
                                          (uintptr_t)w_uv) & 15u ||
       ((uintptr_t)out_latent & 7u) || ((uintptr_t)out_v & 1u))
     return set_error(WS_EINVAL, "ws_mla_merge_split_uv: misaligned buffer");
-  const size_t need = ws::workspace_bytes(Bp, lay.piece_heads, Dv, n_workgroups);
+  const size_t need =
+      ws::workspace_bytes(Bp, lay.piece_heads, Dv, n_workgroups, lay.f32_pieces);
   if (workspace_bytes < need)
     return set_error(WS_EWORKSPACE, "ws_mla_merge_split_uv: workspace %zu < %zu bytes",
                      workspace_bytes, need);
@@ -623,6 +641,7 @@ extern "C" int ws_mla_merge_split_uv(const int32_t* gpu_len, int B, int heads,
   prm.heads = heads;
   prm.Dv = Dv;
   prm.step = lay.step;
+  prm.f32_pieces = lay.f32_pieces;
   prm.cap = page_capacity;
   prm.grid = n_workgroups;
   prm.add = 0;

@@ -48,13 +48,14 @@ struct MlaParams {
   long long c_stride, pe_stride;
   float* out;
   float* lse;
-  uint16_t* part_out;  // [slot][16][512] bf16
-  float* part_lse;     // [slot][16]
+  uint16_t* part_out;  // [slot][hp][512] bf16, or fp32 with f32_pieces
+  float* part_lse;     // [slot][hp]
   // B: plan sequences v = b * ng + g, one per (sequence b, 16-head group g);
   // rows of q / out are v * 16 + h, i.e. b * H + 16 g + h with H = 16 ng.
   // The wide kernel plans sequences (ng = 1) with rows of all H heads.
   int B, ng, page_size, max_pages, num_pages, cap;
   int hp;  // heads of a piece (and of a plan sequence's rows): 16, or all H (wide)
+  bool f32_pieces;  // wide: fp32 pieces (ws_reduce.h mla_layout)
   float scale_log2;
 };
 
@@ -469,7 +470,7 @@ static int mla_launch(const uint16_t* q_nope, const uint16_t* q_pe,
     return set_error(WS_EINVAL, "%s: pools of %lld tokens exceed the 31-bit token index", name,
                      (long long)num_pages * page_size);
   const int n = mla_workgroups(n_workgroups, Bv, max_len);
-  const size_t need = ws::workspace_bytes(Bv, hp, kMlaC, n);
+  const size_t need = ws::workspace_bytes(Bv, hp, kMlaC, n, lay.f32_pieces);
   if (!workspace || workspace_bytes < need)
     return set_error(WS_EWORKSPACE, "%s: workspace %zu < %zu bytes", name, workspace_bytes,
                      need);
@@ -495,6 +496,7 @@ static int mla_launch(const uint16_t* q_nope, const uint16_t* q_pe,
   prm.B = Bv;
   prm.ng = ng;
   prm.hp = hp;
+  prm.f32_pieces = lay.f32_pieces;
   prm.page_size = page_size;
   prm.max_pages = max_pages;
   prm.num_pages = num_pages;

@@ -57,8 +57,9 @@
 // further above m_ref runs again with the true maximum as the reference.
 //
 // Plan (ws_plan.h) over sequences; a sequence held by one workgroup is written
-// final (fp32 out / lse), otherwise each workgroup leaves a bf16 piece of all
-// its heads in slot workgroup + sequence, which the merges combine.  A workgroup that enters a second sequence pays a start and an end
+// final (fp32 out / lse), otherwise each workgroup leaves a piece of all its
+// heads (bf16 or fp32, mla_layout) in slot workgroup + sequence, which the merges
+// combine.  A workgroup that enters a second sequence pays a start and an end
 // again (about 14 us: ten blocks' time), so the plan prefers ranges of one
 // sequence (kAlignStepWide).  128 heads, B = 96 of 256 to 4096 tokens, step and
 // merge: 380 us as eight 16-head groups a sequence, 103 here; B = 40 of 500 to
@@ -669,7 +670,7 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
     // i is column 32 ct + 8 (i / 4) + 4 j2 + i % 4.
     uint32_t* stage = (uint32_t*)&s_tile[0][0] + (size_t)(32 * wave) * 260;
     if (rows == 0) {  // no outputs
-    } else if (!whole) {  // bf16 piece: all 512 columns at once
+    } else if (!whole && !p.f32_pieces) {  // bf16 piece: all 512 columns at once
 #pragma unroll
       for (int ct = 0; ct < 16; ++ct)
 #pragma unroll
@@ -680,8 +681,10 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
       wide_lds_wait();  // this wave's rows are in LDS
       char* dst = (char*)(p.part_out + ((size_t)(g + b) * H + 32 * wave) * kMlaC);
       wide_store_rows(dst, kMlaC * 2, stage + 4 * lane, 16 * lane, rows);
-    } else {  // fp32 final: two halves of 256 columns
-      char* dst = (char*)(p.out + ((size_t)b * H + 32 * wave) * kMlaC);
+    } else {  // fp32 final or piece: two halves of 256 columns
+      float* rows0 = whole ? p.out + (size_t)b * H * kMlaC
+                           : (float*)p.part_out + (size_t)(g + b) * H * kMlaC;
+      char* dst = (char*)(rows0 + 32 * wave * kMlaC);
 #pragma unroll
       for (int hc = 0; hc < 2; ++hc) {
 #pragma unroll

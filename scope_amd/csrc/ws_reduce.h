@@ -10,7 +10,7 @@
 // Workspace layout (ws_decode_plan), for a call over rows_kv rows of `heads`
 // output rows each, run by n splits:
 //   [slot lse f32 x (n + rows_kv) x heads, padded to 256 B]
-//   [slot out bf16 x (n + rows_kv) x heads x Dv]
+//   [slot out bf16 (some wide MLA calls: fp32, mla_layout) x (n + rows_kv) x heads x Dv]
 // (slot = split + row, ws_plan.h).  Pieces are normalised and rounded to
 // bf16 (their weights stay fp32): a 32-token block carries 36 KB of latent
 // and an MLA piece 16 x 512 outputs, so at 256 splits fp32 pieces cost
@@ -30,12 +30,13 @@ __host__ __device__ inline size_t align256(size_t n) { return (n + 255) & ~(size
 
 struct SplitWorkspace {
   float* part_lse;
-  uint16_t* part_out;  // bf16
+  uint16_t* part_out;  // bf16 (f32_pieces calls: the fp32 values' address)
 };
 
-__host__ __device__ inline size_t workspace_bytes(int rows_kv, int heads, int Dv, int n) {
+__host__ __device__ inline size_t workspace_bytes(int rows_kv, int heads, int Dv, int n,
+                                                  bool f32_pieces = false) {
   const size_t slots = (size_t)n + rows_kv;
-  return align256(slots * heads * 4) + slots * heads * Dv * 2;
+  return align256(slots * heads * 4) + slots * heads * Dv * (f32_pieces ? 4 : 2);
 }
 
 __host__ __device__ inline SplitWorkspace carve_workspace(void* base, int rows_kv,
@@ -63,9 +64,17 @@ __host__ __device__ inline SplitWorkspace carve_workspace(void* base, int rows_k
 // B 16 x H 64: 300 tokens 23.5 -> 20.8, 16k 140 -> 62; B 11 x H 96: 300 tokens
 // 26.4 -> 21.3, 16k 148 -> 55.  Below it: B 16 x H 32 of 1000 tokens 19.1 ->
 // 21.5, B 8 x H 64 of 2048 23.2 -> 26.3.
+//
+// The group layout holds more of these calls' rows whole (fp32), having H / 16
+// times the plan sequences; the wide one cuts nearly every row over workgroups.
+// A bf16 piece rounds its outputs once more, which would show in the error
+// against 64 bits (B 128 x H 32 of 2048 tokens: 0.00133 -> 0.00200 of the output's
+// norm), so these calls leave fp32 pieces.  128 heads over at most 64 sequences
+// cut nearly every row in either layout and keep bf16 ones.
 constexpr int kWideHeads = 128;    // heads of the wide kernel's four waves
 constexpr int kWideMinHeads = 32;
 constexpr int kWideMinRows = 1024;  // B * H from which fewer than 128 heads run it
+constexpr int kWideBf16Seqs = 64;  // sequences up to which 128 heads leave bf16 pieces
 constexpr int kWideMaxSeqs = 16 * kMaxSeqs / kWideMinHeads;  // (a call takes B * H / 16 <= kMaxSeqs)
 struct MlaLayout {
   bool wide;
@@ -73,6 +82,7 @@ struct MlaLayout {
   int piece_heads;  // heads of one piece
   int plan_seqs;    // B * ng
   int step;         // the plan's alignment step (ws_plan.h)
+  bool f32_pieces;  // fp32 pieces instead of bf16 ones
 };
 __host__ __device__ inline MlaLayout mla_layout(int B, int H) {
   MlaLayout l;
@@ -81,6 +91,7 @@ __host__ __device__ inline MlaLayout mla_layout(int B, int H) {
   l.piece_heads = l.wide ? H : 16;
   l.plan_seqs = B * l.ng;
   l.step = l.wide ? kAlignStepWide : kAlignStep;
+  l.f32_pieces = l.wide && (H < kWideHeads || B > kWideBf16Seqs);
   return l;
 }
 
@@ -140,20 +151,24 @@ __device__ __forceinline__ float acc_factor(float m, float M) {
   return m == neg_inf() ? 1.f : __expf(m - M);
 }
 
-// Adds the pieces s, s + step, ... (U of them, those below n) to an
-// accumulator: all U lse values and columns are requested before the first is
-// used (past n the last piece again, a cache hit).
-template <int U>
-__device__ __forceinline__ void piece_batch(PieceAcc& x, const uint16_t* pieces, size_t stride,
+// Four columns of a piece as loaded: VT is uint2 (bf16) or float4 (fp32).
+__device__ __forceinline__ float4 piece4_f32(float4 v) { return v; }
+
+// Adds the pieces s, s + step, ... (U of them, those below n; piece s's columns
+// at pieces + s * stride bytes) to an accumulator: all U lse values and columns
+// are requested before the first is used (past n the last piece again, a cache
+// hit).
+template <int U, class VT>
+__device__ __forceinline__ void piece_batch(PieceAcc& x, const char* pieces, size_t stride,
                                             const float* lse, int lstride, int s, int step,
                                             int n) {
   float l[U];
-  uint2 v[U];
+  VT v[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) l[u] = lse[(size_t)min(s + u * step, n - 1) * lstride];
 #pragma unroll
   for (int u = 0; u < U; ++u)
-    v[u] = *(const uint2*)(pieces + (size_t)min(s + u * step, n - 1) * stride);
+    v[u] = *(const VT*)(pieces + (size_t)min(s + u * step, n - 1) * stride);
   float m = x.m;
 #pragma unroll
   for (int u = 0; u < U; ++u) {
@@ -175,17 +190,18 @@ __device__ __forceinline__ void piece_batch(PieceAcc& x, const uint16_t* pieces,
 }
 
 // The pieces first, first + step, ... of a row's n.
-__device__ __forceinline__ PieceAcc piece_stream(const uint16_t* pieces, size_t stride,
+template <class VT>
+__device__ __forceinline__ PieceAcc piece_stream(const char* pieces, size_t stride,
                                                  const float* lse, int lstride, int first,
                                                  int step, int n) {
   PieceAcc x = piece_acc_empty();
   int s = first;
   for (; s + 8 * step < n; s += 16 * step)
-    piece_batch<16>(x, pieces, stride, lse, lstride, s, step, n);
+    piece_batch<16, VT>(x, pieces, stride, lse, lstride, s, step, n);
   if (s + 4 * step < n)
-    piece_batch<8>(x, pieces, stride, lse, lstride, s, step, n);
+    piece_batch<8, VT>(x, pieces, stride, lse, lstride, s, step, n);
   else if (s < n)
-    piece_batch<4>(x, pieces, stride, lse, lstride, s, step, n);
+    piece_batch<4, VT>(x, pieces, stride, lse, lstride, s, step, n);
   return x;
 }
 

@@ -48,6 +48,13 @@ def test_version_and_plan():
         assert 1 <= n <= max(1, -(-rows * -(-L // 32) // 2)) and n <= 4096
     n, _ = ops.decode_plan(1, 8, 16, 8192, 0)
     assert 1 <= n <= 8 * 256 // 4
+    # MLA pieces of all heads: bf16 for 128 heads over at most 64 sequences, fp32
+    # above and for fewer heads (from 1024 rows on; 16-head bf16 pieces below)
+    for B, H, hp, width in ((64, 128, 128, 2), (65, 128, 128, 4), (32, 32, 32, 4), (31, 32, 16, 2),
+                            (10, 112, 112, 4)):
+        n, wsb = ops.decode_plan(1, B, H, 16384, 64)
+        slots = 64 + (B if hp == H else B * H // 16)
+        assert n == 64 and wsb == pad(slots * hp * 4) + slots * hp * 512 * width, (B, H)
     with pytest.raises(ops.WsError):
         ops.decode_plan(0, 16, 0, 100, 0)  # no heads
     with pytest.raises(ops.WsError):

@@ -150,6 +150,38 @@ def test_mla_many_sequences(B, H, wg):
         assert_close(ov[b], torch.einsum("hk,hvk->hv", o, w), OUT_ATOL, OUT_RTOL, f"out_v {b}")
 
 
+@pytest.mark.parametrize("B,H", [(128, 32), (64, 64), (65, 128)])
+def test_mla_many_sequences_round_only_their_probabilities(B, H):
+    """Batches whose rows the one-pass kernel cuts over workgroups: the pieces
+    are fp32, so an output's error is that of bf16 probabilities alone.  Rounding
+    to 8 significant bits errs by up to 2^-8 / m of a value of significand m, in
+    rms over m log-uniform on [1, 2) by 2^-8 / sqrt(3) * sqrt(0.541) = 0.00166, and
+    over random values the output errs by no more.  A bf16 piece adds as much
+    again (0.0020 measured)."""
+    L, scale = 2047, 192 ** -0.5
+    print(f"mla precision B={B} H={H}", flush=True)
+    lat, pt = _pool([L] * B, (PS, 576), 31)
+    qn = bf16_randn((B * H, 512), 32, 0.5).to(DEV)
+    qp = bf16_randn((B * H, 64), 33, 0.5).to(DEV)
+    gl = torch.full((B,), L, dtype=torch.int32, device=DEV)
+    out, _ = ops.mla_decode_partial(qn, qp, lat, pt, gl, scale, L)
+    st = ops.mla_append_decode_split(qn, qp, bf16_randn((B, 1, 512), 34, 0.5).to(DEV),
+                                     bf16_randn((B, 1, 64), 35, 0.5).to(DEV), lat, pt, gl,
+                                     torch.zeros_like(gl), scale, L + 1)
+    merged, _ = ops.merge_split(st, None, out_dtype=torch.float32)
+    q = torch.cat([qn, qp], 1).view(B, H, 576)
+    t = torch.arange(L + 1, device=DEV)
+    for got, n in ((out, L), (merged, L + 1)):
+        err = ref = 0.0
+        for b in range(0, B, 8):
+            x = lat[pt[b, t[:n] // PS].long(), t[:n] % PS].double()
+            w = torch.softmax(torch.matmul(q[b].double(), x.t()) * scale, -1)
+            o = torch.matmul(w, x[:, :512])
+            err += float((got.view(B, H, 512)[b] - o).square().sum())
+            ref += float(o.square().sum())
+        assert (err / ref) ** 0.5 <= 0.00166, (n, (err / ref) ** 0.5)
+
+
 @pytest.mark.parametrize("n,tokens,shape", [(1, 0, (1, 1, 1)), (3, 5, (3, 100, 1)),
                                             (256, 4097, (256, 1, 1)), (2049, 7, (2049, 1, 1)),
                                             (0, 3, (0, 4, 1))])
