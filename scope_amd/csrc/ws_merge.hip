@@ -238,7 +238,8 @@ merge_split_kernel(const MergeSplitParams p) {
   int grp = PS > 1 ? blockIdx.y : blockIdx.y * waves + wave;
   if (PS == 1 && grp >= groups) return;
   // The host partial's address depends on nothing the plan computes: its
-  // loads go out first.
+  // loads go out first, once per column group (of PS waves the first uses them;
+  // the operand may be host memory, read over the link).
   MergeCol mc = merge_col(grp, lane, p.heads, Dv4);
   float lb = neg_inf();
   float4 ob = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -247,7 +248,7 @@ merge_split_kernel(const MergeSplitParams p) {
       load_b<(FMT >= 0 ? FMT : 0)>(p.b_out, p.b_aux0, p.b_aux1, (int)(krow * p.heads + mc.h),
                                    p.Dv, mc.c, lb, ob);
   };
-  host();
+  if (PS == 1 || wave == 0) host();
   const RowSplits rs = plan_row(p.gpu_len, p.add, p.cap, p.B, p.R, p.grid, b, r, p.ng, p.step);
   if (p.in_place && rs.nseg <= 1) return;  // out / lse hold the row
   auto store = [&](const float4& o, float lse) {

@@ -6,6 +6,8 @@ import pytest
 import torch
 
 from scope_amd import ops
+from tests.gpu_pool import mla_pool
+from tests.helpers import bf16_randn
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -68,6 +70,33 @@ def test_merges_read_pinned_host_operands_in_place(fmt):
                                  out_dtype=torch.float32)
         torch.cuda.synchronize()
         assert torch.equal(got, want) and torch.equal(gl, wl), rep
+
+
+@pytest.mark.parametrize("B,wg", [(2, 200), (8, 96), (40, 60)])  # 8, 4 and 1 waves a group
+def test_split_merges_read_pinned_host_operands_in_place(B, wg):
+    """The split step's merges with a pinned operand: the bits of the same merge
+    with the operand on the GPU, whatever the number of waves that share a
+    column group (the first of them reads the operand)."""
+    _say(f"merge_split with a pinned host operand B={B} wg={wg}")
+    H, PS, scale = 16, 64, 192 ** -0.5
+    lens = [3000 + 70 * b for b in range(B)]
+    lat, pt, gl, cs, pes = mla_pool([L + 1 for L in lens], PS, seed=21)
+    gl.copy_(torch.tensor(lens, dtype=torch.int32, device=DEV))
+    qn = bf16_randn((B * H, 512), 22, 0.5).to(DEV)
+    qp = bf16_randn((B * H, 64), 23, 0.5).to(DEV)
+    st = ops.mla_append_decode_split(qn, qp, torch.stack([c[-1:] for c in cs]).to(DEV),
+                                     torch.stack([p[-1:] for p in pes]).to(DEV), lat, pt, gl,
+                                     torch.zeros_like(gl), scale, max(lens) + 1, n_workgroups=wg)
+    hb = (bf16_randn((B * H, 512), 24, 0.1).pin_memory(),
+          (torch.randn(B * H, generator=torch.Generator().manual_seed(25)) + 7).pin_memory())
+    w_uv = bf16_randn((H, 64, 512), 26, 0.05).to(DEV)
+    got, want = ([*ops.merge_split(st, b, ops.PARTIAL_LSE_BF16, out_dtype=torch.float32),
+                  *ops.merge_split_uv(st, w_uv, b, ops.PARTIAL_LSE_BF16, want_latent=True,
+                                      want_lse=True)]
+                 for b in (hb, tuple(x.to(DEV) for x in hb)))
+    torch.cuda.synchronize()
+    for i, (x, y) in enumerate(zip(got, want)):
+        assert torch.equal(x, y) and bool(torch.isfinite(x).all()), i
 
 
 @pytest.mark.parametrize("page_shape,wg", [((64, 576), 0), ((8, 64, 128), 0), ((3, 16), 0),
