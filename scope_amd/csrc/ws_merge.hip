@@ -496,7 +496,8 @@ extern "C" int ws_merge_split(const int32_t* gpu_len, int B, int rows_per_seq, i
   const bool mla = Dv == 512 && rows_per_seq == 1 && heads > 16 && heads % 16 == 0;
   const MlaLayout lay = mla_layout(B, heads);
   const int ng = mla ? lay.ng : 1;
-  if (B < 0 || (long long)B * ng > kMaxSeqs || rows_per_seq <= 0 || heads <= 0 ||
+  // (a step takes at most kMaxSeqs (sequence, 16-head group) pairs in any layout)
+  if (B < 0 || (long long)B * (mla ? heads / 16 : 1) > kMaxSeqs || rows_per_seq <= 0 || heads <= 0 ||
       (heads > 16 && !mla) || Dv <= 0 || Dv % 4 || Dv > 512 || page_capacity <= 0 ||
       n_workgroups <= 0)
     return set_error(WS_EINVAL, "ws_merge_split: bad sizes");

@@ -123,6 +123,19 @@ def test_host_side_argument_checks():
     assert rc == -1 and b"b_aux1" in L.ws_last_error()
     rc = L.ws_lse_merge(fake, fake, fake, fake, None, 9, None, fake, None, 4, 128, None)
     assert rc == -1 and b"format" in L.ws_last_error()
+    # the merges of an MLA step take the step's batch limit, B * heads / 16 <= 2048,
+    # at every head count (a short workspace, rc -3, is looked at afterwards)
+    for B, H in ((257, 128), (2048, 32), (683, 48), (120, 288)):
+        rc = L.ws_merge_split(fake, B, 1, H, 512, 64, 16, fake, fake, fake, 0, None, None, None, 0,
+                              fake, None, None, None)
+        assert rc == -1 and b"bad sizes" in L.ws_last_error(), (B, H)
+        rc = L.ws_mla_merge_split_uv(fake, B, H, 64, 16, fake, fake, fake, 0, None, None, None, 0,
+                                     fake, 128, None, fake, None, None)
+        assert rc == -1 and b"bad sizes" in L.ws_last_error(), (B, H)
+    for B, H in ((256, 128), (1024, 32), (682, 48)):
+        rc = L.ws_merge_split(fake, B, 1, H, 512, 64, 16, fake, fake, fake, 0, None, None, None, 0,
+                              fake, None, None, None)
+        assert rc == -3, (B, H)
     # ws_copy: alignment, size and overlap are checked before any launch
     rc = L.ws_copy(fake, ctypes.c_void_p(0x2008), 64, None)
     assert rc == -1 and b"aligned" in L.ws_last_error()
