@@ -364,9 +364,9 @@ __global__ __launch_bounds__(kUvThreads) void merge_split_uv_kernel(
       if (PS > 1) s_acc[first + i][c] = x;
     }
   if (PS > 1) __syncthreads();
+  float lse = 0.f;
   if (first == 0) {
     float4 o;
-    float lse;
     if constexpr (PS > 1)
       merge_finish([&](int i) { return s_acc[i][c]; }, PS, lb, ob, o, lse);
     else
@@ -375,13 +375,14 @@ __global__ __launch_bounds__(kUvThreads) void merge_split_uv_kernel(
     packed.x = pack_bf16x2(o.x, o.y);
     packed.y = pack_bf16x2(o.z, o.w);
     if (p.out_bf16) ((uint2*)(p.out_bf16 + (size_t)qrow * Dv))[c] = packed;
-    if (p.lse_out && c == 0) p.lse_out[qrow] = lse;
     s_row[4 * c + 0] = bf16_to_f32(packed.x & 0xffffu);
     s_row[4 * c + 1] = bf16_to_f32(packed.x >> 16);
     s_row[4 * c + 2] = bf16_to_f32(packed.y & 0xffffu);
     s_row[4 * c + 3] = bf16_to_f32(packed.y >> 16);
   }
   __syncthreads();
+  // (here, where both waves have read the row's lse_g: lse_out may be lse_g)
+  if (p.lse_out && t == 0) p.lse_out[qrow] = lse;
   // out_v[b][h * Dout + v] = sum_k s_row[k] * W_UV[h][v][k]: eight lanes per
   // W_UV row, kUvThreads / 8 rows per pass, kUvGroup passes per group of loads
   for (int v0 = 0; v0 < Dout; v0 += kUvGroup * (kUvThreads / 8)) {

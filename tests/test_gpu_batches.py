@@ -182,6 +182,34 @@ def test_mla_many_sequences_round_only_their_probabilities(B, H):
         assert (err / ref) ** 0.5 <= 0.00166, (n, (err / ref) ** 0.5)
 
 
+@pytest.mark.parametrize("L,wg", [(60, 0), (3000, 12), (3000, 200)])  # whole rows, 1, 4 waves
+def test_uv_merge_writes_its_lse_over_the_steps(L, wg):
+    """lse_out may be the step's lse_g: both waves of a row read it before either
+    result is written.  The bits of the merge with buffers of its own."""
+    B, H, scale = 24, 16, 192 ** -0.5
+    print(f"uv merge in place L={L} wg={wg}", flush=True)
+    lat, pt = _pool([L] * B, (PS, 576), 41)
+    gl = torch.full((B,), L, dtype=torch.int32, device=DEV)
+    st = ops.mla_append_decode_split(bf16_randn((B * H, 512), 42, 0.5).to(DEV),
+                                     bf16_randn((B * H, 64), 43, 0.5).to(DEV),
+                                     bf16_randn((B, 1, 512), 44, 0.5).to(DEV),
+                                     bf16_randn((B, 1, 64), 45, 0.5).to(DEV), lat, pt, gl,
+                                     torch.zeros_like(gl), scale, L + 1, n_workgroups=wg)
+    w_uv = bf16_randn((H, 32, 512), 46, 0.05).to(DEV)
+    ho = bf16_randn((B * H, 512), 47, 0.1).to(DEV)
+    hl = torch.full((B * H,), 7.0, device=DEV)
+    want, _, wl = ops.merge_split_uv(st, w_uv, (ho, hl), ops.PARTIAL_LSE_BF16, want_lse=True)
+    got = torch.empty_like(want)
+    ws = st.workspace
+    rc = ops.lib().ws_mla_merge_split_uv(
+        st.gpu_len.data_ptr(), B, H, st.cap, st.nwg, st.out_g.data_ptr(), st.lse_g.data_ptr(),
+        ws.data_ptr(), ws.numel(), ho.data_ptr(), hl.data_ptr(), None, ops.PARTIAL_LSE_BF16,
+        w_uv.data_ptr(), 32, None, got.data_ptr(), st.lse_g.data_ptr(),
+        torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert rc == 0 and torch.equal(got, want) and torch.equal(st.lse_g.view(-1), wl)
+
+
 @pytest.mark.parametrize("n,tokens,shape", [(1, 0, (1, 1, 1)), (3, 5, (3, 100, 1)),
                                             (256, 4097, (256, 1, 1)), (2049, 7, (2049, 1, 1)),
                                             (0, 3, (0, 4, 1))])
