@@ -295,7 +295,8 @@ static void launch_merge(const MergeSplitParams& p, long long rows, hipStream_t 
     hipLaunchKernelGGL((merge_split_kernel<FMT, 4, uint2>), dim3((unsigned)rows, groups), dim3(256),
                        0, s, p);
   } else {
-    const int waves = std::min(groups, kMergeWgWaves);
+    // (a grid dimension holds fewer than 2^32 threads: two waves at 2^24 rows)
+    const int waves = std::min(groups, rows < (1LL << 32) / (64 * kMergeWgWaves) ? kMergeWgWaves : 2);
     const long long fit = std::max(kMergeWaves / (rows * waves), 1LL);
     const int wgs = (int)std::min<long long>((groups + waves - 1) / waves, fit);
     const dim3 grid((unsigned)rows, wgs), block(64 * waves);
