@@ -1,7 +1,8 @@
 """Absorbed MLA with more than 16 heads on the GPU (DeepSeek-V2: 128 heads
 over one shared 576-wide latent; the reference takes nH = q rows / B,
 kernel/cpu_attn.cpp:860, system/deepseek.py:256-260): each 16-head group is a
-plan sequence of its own over the same latent.  Against fp64, through the
+plan sequence of its own over the same latent, and larger batches run one pass
+over it for all heads.  Against fp64, through the
 one-launch partial, the split step with the native host partial and the
 merge, the merge with the W_UV epilogue, and the paged two-sided cache.
 """
@@ -305,3 +306,99 @@ def test_mla_128_heads_b4_full_size_against_the_c_restatement():
                                                   n_threads=16)
         assert_close(out[rows], po / ps[:, None], OUT_ATOL, OUT_RTOL, f"out b={b} vs C port")
         assert_close(lse[rows], pm + np.log(ps), LSE_ATOL, LSE_RTOL, f"lse b={b} vs C port")
+
+
+# Head counts between 16 and 128 at batches that run the one-pass kernel (B * H
+# >= 1024): full, half-filled and empty 32-head waves (32: 1 + 0, 48: 1 + 1/2 + 2
+# empty, 112: 3 + 1/2).
+ONE_PASS = [(32, 32), (48, 22), (112, 10)]
+
+
+def _one_pass_case(H, B, seed, factor=1.0):
+    """Sequences of up to 2500 tokens (79 blocks) and one more each to append;
+    factor scales the rope keys after the first 32 tokens."""
+    lens = [(2500, 40, 97, 0, 64)[b % 5] for b in range(B)]
+    lens[-1] = 2200
+    rows = []
+    for b, L in enumerate(lens):
+        x = bf16_randn((L + 1, 576), seed + b, 0.5).float()
+        x[32:, 512:] *= factor
+        rows.append(x.to(torch.bfloat16))
+    lat, pt, gl, _, _ = mla_pool([L + 1 for L in lens], PS, seed=seed)
+    for b, L in enumerate(lens):
+        t = torch.arange(L, device=DEV)
+        lat[pt[b, t // PS].long(), t % PS] = rows[b][:L].to(DEV)
+    gl.copy_(torch.tensor(lens, dtype=torch.int32, device=DEV))
+    qn = bf16_randn((B * H, 512), seed + 700, 0.5).to(DEV)
+    qp = bf16_randn((B * H, 64), seed + 701, 0.5).to(DEV)
+    new = torch.stack([x[-1] for x in rows]).to(DEV)[:, None]
+    return lens, rows, lat, pt, gl, qn, qp, new
+
+
+def _check_one_pass(H, rows, scale, qn, qp, out, lse, seqs, what):
+    out, lse = out.cpu().numpy(), lse.cpu().numpy()
+    for b in seqs:
+        at = slice(b * H, (b + 1) * H)
+        want, wl = O.mla_attention_fp64(bits(qn[at]), bits(qp[at]), bits(rows[b][:, :512])[None],
+                                        bits(rows[b][:, 512:])[None], scale)
+        assert_close(out[at], want, OUT_ATOL, OUT_RTOL, f"{what} b={b} out")
+        assert_close(lse[at], wl, LSE_ATOL, LSE_RTOL, f"{what} b={b} lse")
+
+
+@pytest.mark.parametrize("H,B", ONE_PASS)
+@pytest.mark.parametrize("factor,wg", [(1.0, 3), (1024.0, 3), (1024.0, 0)])
+def test_one_pass_heads_climbing_scores_and_long_segments(H, B, factor, wg):
+    """Scores that climb out of the first block's range (the segment runs again,
+    the waves without heads with it) and segments of more than 64 blocks (the
+    page window is fetched again), with the fused append and without."""
+    _say(f"one pass H={H} B={B} factor={factor} wg={wg}")
+    lens, rows, lat, pt, gl, qn, qp, new = _one_pass_case(H, B, 900, factor)
+    out, lse = ops.mla_decode_partial(qn, qp, lat, pt, gl, SCALE, max(lens), n_workgroups=wg)
+    _check_one_pass(H, [x[:-1] for x in rows], SCALE, qn, qp, out, lse, range(B), "old tokens")
+    len_out = torch.zeros_like(gl)
+    out, lse = ops.mla_append_decode_partial(qn, qp, new[..., :512], new[..., 512:], lat, pt, gl,
+                                             len_out, SCALE, max(lens) + 1, n_workgroups=wg)
+    _check_one_pass(H, rows, SCALE, qn, qp, out, lse, range(B), "appended")
+    assert len_out.cpu().tolist() == [L + 1 for L in lens]
+    lb = bits(lat)
+    for b, L in enumerate(lens):
+        assert np.array_equal(lb[int(pt[b, L // PS]), L % PS], bits(rows[b][-1])), b
+
+
+@pytest.mark.parametrize("H,B", ONE_PASS)
+@pytest.mark.parametrize("scale", [-SCALE, 0.0])
+def test_one_pass_heads_non_positive_scale(H, B, scale):
+    _say(f"one pass H={H} B={B} scale={scale}")
+    lens, rows, lat, pt, gl, qn, qp, new = _one_pass_case(H, B, 1000)
+    out, lse = ops.mla_append_decode_partial(qn, qp, new[..., :512], new[..., 512:], lat, pt, gl,
+                                             None, scale, max(lens) + 1, n_workgroups=7)
+    _check_one_pass(H, rows, scale, qn, qp, out, lse, range(B), f"scale {scale}")
+
+
+@pytest.mark.parametrize("H,B", ONE_PASS)
+@pytest.mark.parametrize("bad_new_page", [False, True])
+def test_one_pass_heads_poison_bad_pages_and_lengths(H, B, bad_new_page):
+    """A page id outside the pool, the appended token's own page among them, and
+    invalid lengths poison their sequence's rows (NaN, len_out -1 for a length)
+    and no other's; nothing is written where a clamped id points."""
+    _say(f"one pass H={H} B={B} poison bad_new_page={bad_new_page}")
+    lens, rows, lat, pt, gl, qn, qp, new = _one_pass_case(H, B, 1100)
+    pt[0, lens[0] // PS if bad_new_page else 3] = -5  # read as pool page 0
+    gl[2], gl[4] = 10 ** 6, -2
+    before = bits(lat[0, lens[0] % PS])
+    len_out = torch.zeros_like(gl)
+    st = ops.mla_append_decode_split(qn, qp, new[..., :512], new[..., 512:], lat, pt, gl, len_out,
+                                     SCALE, max(lens) + 1, n_workgroups=5)
+    host = (torch.zeros((B * H, 512), device=DEV),
+            torch.full((B * H,), float("-inf"), device=DEV))
+    out, lse = ops.merge_split(st, host, ops.PARTIAL_LSE_F32, out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    bad = (0, 2, 4)
+    _check_one_pass(H, rows, SCALE, qn, qp, out, lse, [b for b in range(B) if b not in bad],
+                    "beside poisoned ones")
+    o, l = out.view(B, H, 512).cpu(), lse.view(B, H).cpu()
+    for b in bad:
+        assert bool(torch.isnan(o[b]).all()) and bool(torch.isnan(l[b]).all()), b
+    assert len_out.cpu().tolist() == [-1 if b in (2, 4) else L + 1 for b, L in enumerate(lens)]
+    if bad_new_page and 0 not in [int(pt[b, L // PS]) for b, L in enumerate(lens) if b]:
+        assert np.array_equal(bits(lat[0, lens[0] % PS]), before)

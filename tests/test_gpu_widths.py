@@ -221,6 +221,16 @@ def test_gqa_width_split_step_and_host_merge(D, fmt):
         assert_close(gls[b], wl, LSE_ATOL, LSE_RTOL, f"merged lse D={D} b={b}")
 
 
+@pytest.mark.parametrize("D", [144, 160, 192])
+def test_gqa_widths_with_two_key_stages_and_one_value_stage(D):
+    """The widths whose ring requests a block's values under the next block's
+    scores, through every step that appends: the appended row's values are
+    stored from the one value stage before it is requested again."""
+    test_gqa_width_fused_steps_append_bit_exact(D)
+    test_gqa_width_full_step_bf16(D)
+    test_gqa_width_split_step_and_host_merge(D, ops.PARTIAL_LSE_F32)
+
+
 @pytest.mark.parametrize("D", WIDTHS + [80])
 def test_gqa_width_noalloc_matches_workspace_call(D):
     """The no-allocation entry point at another width: bit-identical to the
