@@ -149,17 +149,19 @@ int ws_dense_paging(int32_t* page_table, int32_t* gpu_len, int n, int tokens, fl
  * Plan of a decode call: kind 0 (GQA: rows_kv = B * Hkv, heads = the group
  * size G) or 1 (MLA: rows_kv = B, heads = H, a multiple of 16; H = 128, and
  * 32 <= H < 128 from B * H = 1024, plan sequences with H-head pieces, others
- * 16-head groups), over sequences of at most max_len tokens.  n_splits is the number of pieces the call cuts its work
- * into: one per wave for GQA (two per workgroup, each streaming on its
+ * 16-head groups), over sequences of at most max_len tokens.  n_splits is the
+ * number of pieces the call cuts its work into: one per wave for GQA (two per workgroup, each streaming on its
  * own), one per workgroup for MLA.  0 = the library's choice for the current
  * device: two GQA waves (one workgroup) or one MLA workgroup per CU, fewer
- * when the batch is small (a GQA split keeps at least two 32-token blocks).  Writes the resolved split count and the
- * workspace bytes the call needs; the same count goes to ws_merge_split.
+ * when the batch is small (a GQA split keeps at least two 32-token blocks).
+ * Writes the resolved split count and the workspace bytes the call needs; the
+ * same count goes to ws_merge_split.
  *
  * Splits take equal shares of all 32-token blocks of all rows, so ragged
  * batches stay balanced; a row shared by several splits is combined from
  * their partials.  Workspace layout: [partial lse fp32, padded to 256
- * bytes][partial out bf16], one partial slot per (split, row) pair.  The
+ * bytes][partial out bf16, or fp32 (MLA pieces of H heads, except 128 heads over
+ * at most 64 sequences)], one partial slot per (split, row) pair.  The
  * workspace must be 256-byte aligned; it needs no initial contents (every
  * call writes the slots it reads back).  Calls that share a workspace must
  * be ordered on one stream.  At most 2048 sequences and 4096 splits per

@@ -563,9 +563,9 @@ static int gqa_launch(const uint16_t* q, const uint16_t* k_new, const uint16_t* 
                      name, (long long)B * Hkv, max_len);
   const int rows_kv = B * Hkv;
   const int n = gqa_splits(n_splits, rows_kv, max_len, D);
-  if (n > kReduceMaxWeights)
+  if (n > kMaxSplits)
     return set_error(WS_EINVAL, "%s: %d splits exceed the merge's %d", name, n,
-                     kReduceMaxWeights);
+                     kMaxSplits);
   const size_t need = ws::workspace_bytes(rows_kv, G, D, n);
   if (!workspace || workspace_bytes < need)
     return set_error(WS_EWORKSPACE, "%s: workspace %zu < %zu bytes", name, workspace_bytes,

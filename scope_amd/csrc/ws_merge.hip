@@ -1,8 +1,11 @@
-// LSE merge of the GPU partial with a second (host) partial, fused with the
-// final normalisation and the bf16 cast.  One workgroup per row, one float4
-// of the output per thread.  The second operand may arrive in any of the
-// reference CPU kernels' output conventions, so no conversion launch is
-// needed after its host-to-device copy.
+// LSE merges, fused with the final normalisation and the bf16 cast:
+//   lse_merge_kernel       a GPU partial with a second (host) partial: one
+//                          workgroup per row, one float4 of the output per thread
+//   merge_split_kernel     a split step's pieces, with or without a host partial
+//   merge_split_uv_kernel  the same of an absorbed-MLA step, through W_UV
+// The host partial may arrive in any of the reference CPU kernels' output
+// conventions, so no conversion launch is needed after its host-to-device copy,
+// and may be pinned host memory, read in place.
 #include <math.h>
 
 #include <algorithm>
@@ -132,9 +135,18 @@ struct MergeSplitParams {
 
 // Waves that share a column group: 1, or more where the rows have many pieces
 // on average (n splits over rows plan rows, about n / rows + 1 each) and the
-// column groups alone do not fill the chip: with eight waves on each of 1024
-// groups of 64 pieces (4 sequences x 128 heads x 512 columns) the merge took
-// 11.0 us, with one 9.4; on 16 groups of 64 pieces 4.6 against 6.8.
+// column groups alone do not fill the chip.  Merge launches alone, captured, us
+// with 1 / 2 / 4 / 8 waves (the rule's choice in brackets):
+//     16 groups of 64 pieces    9.4   5.9   4.9  [4.5]
+//    256 groups of 256         16.0   8.7   6.4  [5.6]
+//    256 groups of 32           6.5   4.5   4.0  [4.2]
+//    512 groups of 64           5.1   4.3  [4.2]  5.0
+//   1024 groups of 64          11.0   8.3  [7.6]  8.8
+//   1024 groups of 8            4.0   4.0  [4.8]  6.6
+//   2048 groups of 32          [7.6]  7.2   7.8  11.2
+//  12288 groups of 2 to 3     [18.9] 36.0  61.6 123
+// 1024 groups of 8 equal pieces alone would do with one; ragged batches of that
+// average have rows of dozens.
 constexpr int kMergeMaxStreams = 8;
 static int merge_streams(int n, long long rows, int groups) {
   if (n >= 24 * rows && rows * groups <= 512) return kMergeMaxStreams;
@@ -296,7 +308,8 @@ static void launch_merge(const MergeSplitParams& p, long long rows, hipStream_t 
                        0, s, p);
   } else {
     // (a grid dimension holds fewer than 2^32 threads: two waves at 2^24 rows)
-    const int waves = std::min(groups, rows < (1LL << 32) / (64 * kMergeWgWaves) ? kMergeWgWaves : 2);
+    const int most = rows * 64 * kMergeWgWaves < (1LL << 32) ? kMergeWgWaves : 2;
+    const int waves = std::min(groups, most);
     const long long fit = std::max(kMergeWaves / (rows * waves), 1LL);
     const int wgs = (int)std::min<long long>((groups + waves - 1) / waves, fit);
     const dim3 grid((unsigned)rows, wgs), block(64 * waves);
@@ -499,8 +512,8 @@ extern "C" int ws_merge_split(const int32_t* gpu_len, int B, int rows_per_seq, i
   const MlaLayout lay = mla_layout(B, heads);
   const int ng = mla ? lay.ng : 1;
   // (a step takes at most kMaxSeqs (sequence, 16-head group) pairs in any layout)
-  if (B < 0 || (long long)B * (mla ? heads / 16 : 1) > kMaxSeqs || rows_per_seq <= 0 || heads <= 0 ||
-      (heads > 16 && !mla) || Dv <= 0 || Dv % 4 || Dv > 512 || page_capacity <= 0 ||
+  if (B < 0 || (long long)B * (mla ? heads / 16 : 1) > kMaxSeqs || rows_per_seq <= 0 ||
+      heads <= 0 || (heads > 16 && !mla) || Dv <= 0 || Dv % 4 || Dv > 512 || page_capacity <= 0 ||
       n_workgroups <= 0)
     return set_error(WS_EINVAL, "ws_merge_split: bad sizes");
   const int Bp = B * ng;      // plan sequences
@@ -509,9 +522,9 @@ extern "C" int ws_merge_split(const int32_t* gpu_len, int B, int rows_per_seq, i
     return set_error(WS_EINVAL, "ws_merge_split: host partial without its lse / max / sum");
   if (b_out && !fmt_known(fmt_b))
     return set_error(WS_EINVAL, "ws_merge_split: unknown format %d", fmt_b);
-  if (n_workgroups > kReduceMaxWeights)
+  if (n_workgroups > kMaxSplits)
     return set_error(WS_EINVAL, "ws_merge_split: %d workgroups exceed %d", n_workgroups,
-                     kReduceMaxWeights);
+                     kMaxSplits);
   if (((uintptr_t)workspace & 255u) || ((uintptr_t)out_g | (uintptr_t)out_f32 |
                                          (uintptr_t)b_out) & 15u || ((uintptr_t)out_bf16 & 7u))
     return set_error(WS_EINVAL, "ws_merge_split: misaligned buffer");
@@ -622,9 +635,9 @@ extern "C" int ws_mla_merge_split_uv(const int32_t* gpu_len, int B, int heads,
     return set_error(WS_EINVAL, "ws_mla_merge_split_uv: host partial without its lse / max / sum");
   if (b_out && !fmt_known(fmt_b))
     return set_error(WS_EINVAL, "ws_mla_merge_split_uv: unknown format %d", fmt_b);
-  if (n_workgroups > kReduceMaxWeights)
+  if (n_workgroups > kMaxSplits)
     return set_error(WS_EINVAL, "ws_mla_merge_split_uv: %d workgroups exceed %d", n_workgroups,
-                     kReduceMaxWeights);
+                     kMaxSplits);
   if (((uintptr_t)workspace & 255u) || ((uintptr_t)out_g | (uintptr_t)b_out |
                                          (uintptr_t)w_uv) & 15u ||
       ((uintptr_t)out_latent & 7u) || ((uintptr_t)out_v & 1u))

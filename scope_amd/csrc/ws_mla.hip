@@ -415,13 +415,12 @@ static bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 // Workgroups of an MLA call: n_workgroups when given, else one per CU (the
 // kernel's occupancy), at most what the blocks of the longest possible batch
 // can feed with 4 blocks each, or one per plan sequence (B) where that is more
-// (sequences of one to three blocks), and no more than the reduction's weights
-// hold.
+// (sequences of one to three blocks), and no more than the plan takes.
 int mla_workgroups(int n_workgroups, int B, int max_len) {
   if (n_workgroups > 0) return n_workgroups;
   const long long max_blocks = (long long)B * std::max((max_len + 31) / 32, 4);
   const int n = choose_workgroups(0, 1, max_blocks, 4);
-  return std::min(n, kReduceMaxWeights);
+  return std::min(n, kMaxSplits);
 }
 
 static int mla_launch(const uint16_t* q_nope, const uint16_t* q_pe,
@@ -449,9 +448,9 @@ static int mla_launch(const uint16_t* q_nope, const uint16_t* q_pe,
     return set_error(WS_EINVAL,
                      "%s: bad paging page_size=%d max_pages=%d num_pages=%d max_len=%d",
                      name, page_size, max_pages, num_pages, max_len);
-  if (n_workgroups < 0 || n_workgroups > kReduceMaxWeights)
+  if (n_workgroups < 0 || n_workgroups > kMaxSplits)
     return set_error(WS_EINVAL, "%s: n_workgroups %d outside [0, %d]", name, n_workgroups,
-                     kReduceMaxWeights);
+                     kMaxSplits);
   if (!aligned16(q_nope) || !aligned16(q_pe) || !aligned16(latent_pages) ||
       !aligned16(out))
     return set_error(WS_EINVAL, "%s: buffers must be 16-byte aligned", name);

@@ -62,7 +62,7 @@
 // combine.  A workgroup that enters a second sequence pays a start and an end
 // again (about 14 us: ten blocks' time), so the plan prefers ranges of one
 // sequence (kAlignStepWide).  128 heads, B = 96 of 256 to 4096 tokens, step and
-// merge: 380 us as eight 16-head groups a sequence, 103 here; B = 40 of 500 to
+// merge: 380 us as eight 16-head groups a sequence, 106 here; B = 40 of 500 to
 // 4000 tokens 75 -> 59 us by the alignment.
 #pragma once
 
@@ -336,7 +336,8 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
       }
 #pragma unroll
       for (int u = 32; u < 36; ++u)
-        qb[u] = ((const u32x4*)(p.q_pe + ((size_t)b * H + min(head, H - 1)) * 64))[2 * (u - 32) + j2];
+        qb[u] =
+            ((const u32x4*)(p.q_pe + ((size_t)b * H + min(head, H - 1)) * 64))[2 * (u - 32) + j2];
       asm volatile("s_waitcnt vmcnt(0)" : "+v"(raw_pid), "+v"(new_pid) : : "memory");
       set_pids(raw_pid);
       if (new_pid >= 0 && new_pid < p.num_pages)

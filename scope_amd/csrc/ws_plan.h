@@ -19,10 +19,13 @@ namespace ws {
 
 // Most sequences a call takes (the per-sequence prefix lives in LDS).
 constexpr int kMaxSeqs = 2048;
+// Most splits a call takes: plan_start's products stay below 2^24, plan_align's
+// counts within 16 bits, and plan_owner's quotients exact.
+constexpr int kMaxSplits = 4096;
 
 struct Plan {
   int T;  // total blocks (the host keeps it below 2^31 / grid)
-  int n;  // workgroups with work (min(grid, T)), at most 4096
+  int n;  // workgroups with work (min(grid, T)), at most kMaxSplits
   int q, r;  // T = q n + r
   // The calling split's range [begin, end) and the sequence of block `begin`.
   bool has_work;
@@ -91,9 +94,11 @@ __device__ __forceinline__ int plan_start(const Plan& p, int g) {
   return g * p.q + (int)((unsigned)(g * p.r) / (unsigned)p.n);
 }
 
-// Splits of a sequence of nb blocks at M blocks per split (rM = 1 / M): ceil(nb
-// / M), or one more where the product rounds up; at least 1 and at most nb for
-// nb > 0, and the same in every kernel.
+// Splits of a sequence of nb blocks at M blocks per split (rM: v_rcp_f32's 1 / M,
+// good to an ulp): ceil(nb / M), or one fewer where nb - 1 is a multiple of M and
+// the product rounds below it (a split then takes M + 1 blocks).  At least 1 and
+// at most nb for nb > 0 (nb < 2^19), and the same in every kernel, which is what
+// the plan needs.
 __device__ __forceinline__ int plan_nsplits(int nb, float rM) {
   return nb > 0 ? (int)((float)(nb - 1) * rM) + 1 : 0;
 }

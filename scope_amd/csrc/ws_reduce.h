@@ -23,9 +23,6 @@
 
 namespace ws {
 
-// Most (partial, row) weights one reduction keeps in LDS.
-constexpr int kReduceMaxWeights = 4096;
-
 __host__ __device__ inline size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 struct SplitWorkspace {
@@ -57,13 +54,17 @@ __host__ __device__ inline SplitWorkspace carve_workspace(void* base, int rows_k
 // and read a block once per group.  The step, the merges and the workspace
 // query of a call all take their layout from here, so they agree.
 //
-// 128 heads always run wide.  Fewer do from B * H = 1024 on (in front of that
-// line the wide kernel's longer start and end cost more than the repeated
-// reads).  Step kernel with its reduce, group layout -> wide, ragged lengths up
-// to the given one: B 32 x H 32: 300 tokens 23.4 -> 21.2 us, 4k 53.7 -> 42.3;
-// B 16 x H 64: 300 tokens 23.5 -> 20.8, 16k 140 -> 62; B 11 x H 96: 300 tokens
-// 26.4 -> 21.3, 16k 148 -> 55.  Below it: B 16 x H 32 of 1000 tokens 19.1 ->
-// 21.5, B 8 x H 64 of 2048 23.2 -> 26.3.
+// 128 heads always run wide.  Fewer do from B * H = 1024 on: the wide kernel has
+// a longer start and end per sequence, the group layout reads every block H / 16
+// times.  Captured steps with their merge, equal lengths, us, group -> wide:
+//   B  32 x H 32   64 tokens 11.5 -> 15.6   1001 25.5 -> 29.1   4096 59.0 -> 45.6
+//   B  16 x H 64   64 tokens 11.9 -> 15.8   1001 23.1 -> 27.2  16384 142 -> 83
+//   B 128 x H 32   64 tokens 17.5 -> 20.5   1001 60.3 -> 48.1
+//   B  64 x H 96   64 tokens 26.9 -> 20.3   1001 92.6 -> 47.7
+//   B 512 x H 32   64 tokens 46.7 -> 38.8   1001  226 -> 149
+// so short contexts lose 3 to 5 us near the line and longer ones gain up to half.
+// The line is on rows alone because the merges, which must agree, know no bound
+// on the lengths.  Below it: B 8 x H 64 of 2048 tokens 23.2 -> 26.3.
 //
 // The group layout holds more of these calls' rows whole (fp32), having H / 16
 // times the plan sequences; the wide one cuts nearly every row over workgroups.
@@ -75,7 +76,8 @@ constexpr int kWideHeads = 128;    // heads of the wide kernel's four waves
 constexpr int kWideMinHeads = 32;
 constexpr int kWideMinRows = 1024;  // B * H from which fewer than 128 heads run it
 constexpr int kWideBf16Seqs = 64;  // sequences up to which 128 heads leave bf16 pieces
-constexpr int kWideMaxSeqs = 16 * kMaxSeqs / kWideMinHeads;  // (a call takes B * H / 16 <= kMaxSeqs)
+// (a call takes B * H / 16 <= kMaxSeqs)
+constexpr int kWideMaxSeqs = 16 * kMaxSeqs / kWideMinHeads;
 struct MlaLayout {
   bool wide;
   int ng;           // plan sequences per sequence
@@ -86,7 +88,8 @@ struct MlaLayout {
 };
 __host__ __device__ inline MlaLayout mla_layout(int B, int H) {
   MlaLayout l;
-  l.wide = H == kWideHeads || (H >= kWideMinHeads && H < kWideHeads && (long long)B * H >= kWideMinRows);
+  l.wide = H == kWideHeads ||
+           (H >= kWideMinHeads && H < kWideHeads && (long long)B * H >= kWideMinRows);
   l.ng = l.wide ? 1 : H / 16;
   l.piece_heads = l.wide ? H : 16;
   l.plan_seqs = B * l.ng;

@@ -12,6 +12,7 @@
 namespace ws {
 
 constexpr int kSplitChunk4 = 64;  // float4 columns per workgroup
+constexpr int kReduceMaxWeights = 4096;  // most split weights of a row (16 KB of LDS)
 
 __global__ __launch_bounds__(64) void split_reduce_kernel(
     const float* __restrict__ part_out, const float* __restrict__ part_lse,
