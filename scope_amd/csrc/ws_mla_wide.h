@@ -154,6 +154,14 @@ __device__ __forceinline__ void wide_dma16_add(uint32_t off, const void* sbase,
                : "memory", "scc");
 }
 
+// The largest of three (one NaN: of the others), without the quieting operations
+// the compiler puts in front of fmaxf on what inline assembly computed.
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  float d;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+  return d;
+}
+
 // Waits until at most N vector memory operations of this wave are in flight
 // and its LDS reads are done, then joins the workgroup barrier.
 template <int N>
@@ -427,7 +435,7 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
 
     f32x16 acc[16];
     float m_run = neg_inf();  // reference max (m_ref) of the lane's head
-    float m_max = neg_inf();  // the lane's largest score of the segment so far
+    float m_max = neg_inf();  // the lane's largest raw score (without sx) so far
     float l_run = 0.f;  // the lane's sum of probabilities as rounded
     float s_run = 0.f;  // and in fp32
 
@@ -439,7 +447,8 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
     //            feeds the headroom check, so no lanes are combined except to
     //            set m_run at the pass's first block
     //   soft_p   one dword of a k-step's P^T from its scores (two exp2
-    //            against m_run)
+    //            against m_run), which become the probabilities in fp32
+    //   soft_s   the block's fp32 probabilities added to the lse's sum
     //   PV(k)    MFMA m (k-step m / 16, columns 32 (m % 16) ..) into
     //            accumulator m % 16, its V^T operand from two transposed reads
     //            (tokens 16 s + 8 t + 4 j2 + e, t = 0, 1) three MFMAs ahead
@@ -492,18 +501,17 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) v[i] = 8 * (i >> 2) + (i & 3) < lim ? v[i] : neg_inf();
       }
-      float r = v[0];
+      float r = max3(v[0], v[1], v[2]);
 #pragma unroll
-      for (int i = 1; i < 16; ++i) r = fmaxf(r, v[i]);
-      const float bm = r * sx;
-      m_max = fmaxf(m_max, bm);
+      for (int i = 3; i < 15; i += 2) r = max3(r, v[i], v[i + 1]);
+      m_max = max3(r, v[15], m_max);
       // The pass's first block (first): m_run, unless a second pass set it,
       // becomes the head's largest score.  That block holds at least one
       // token, so for finite inputs m_run is finite from then on and later
       // blocks need not look.
       if (first) {
         float lo, hi;
-        pair_xor32(bm, lo, hi);
+        pair_xor32(m_max * sx, lo, hi);
         m_run = m_run == neg_inf() ? fmaxf(lo, hi) : m_run;
       }
       const float nm = -m_run;
@@ -514,18 +522,21 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
       }
     };
     // soft_p: one dword of a k-step's P^T (two exp2), its two probabilities
-    // added to the row sums: as rounded (the values the PV MFMAs see), which
-    // normalises the outputs, and in fp32 for the lse
-    auto soft_p = [&](const float (&xs)[8], u32x4& pbs, int dd) __attribute__((always_inline)) {
+    // added to the row sum that normalises the outputs as rounded (the values
+    // the PV MFMAs see); soft_s adds them in fp32 for the lse
+    auto soft_p = [&](float (&xs)[8], u32x4& pbs, int dd) __attribute__((always_inline)) {
       typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-      const float p0 = __builtin_amdgcn_exp2f(xs[2 * dd]);
-      const float p1 = __builtin_amdgcn_exp2f(xs[2 * dd + 1]);
-      const uint32_t pk = pack_bf16x2(p0, p1);
-      s_run += p0 + p1;
+      xs[2 * dd] = __builtin_amdgcn_exp2f(xs[2 * dd]);
+      xs[2 * dd + 1] = __builtin_amdgcn_exp2f(xs[2 * dd + 1]);
+      const uint32_t pk = pack_bf16x2(xs[2 * dd], xs[2 * dd + 1]);
       pbs[dd] = pk;
       l_run = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, pk),
                                               __builtin_bit_cast(bf16x2_t, 0x3f803f80u), l_run,
                                               false);
+    };
+    auto soft_s = [&](const float (&xa)[8], const float (&xh)[8]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) s_run += xa[i] + xh[i];
     };
 
     // Step kk of the ring, software-pipelined.  Block kk's scores (xa, xh)
@@ -534,8 +545,10 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
     // the first k-step's probabilities (soft_p from xa), then 24 PV MFMAs,
     // three to every four links (the XDL unit alternates between the
     // independent PV MFMAs and the dependent QK chain), the second k-step's
-    // probabilities beside PV's first k-step; soft_x of block kk + 1 runs
-    // beside the last 8 PV MFMAs.  Block kk + 3's ten load instructions go
+    // probabilities beside PV's first k-step; soft_s and soft_x of block kk + 1
+    // run beside the last 8 PV MFMAs, behind the first of them (the compiler put
+    // the sums in front of all eight, where the matrix unit waited: 4 sequences
+    // of 32k tokens 49.9 us against 49.7).  Block kk + 3's ten load instructions go
     // out over the chain into tile (kk + 3) % 4.  The step waits for block
     // kk + 1 (block kk + 2 may be in flight) and the barrier (every wave's
     // part of block kk + 1 is in, every wave is done with step kk - 1 and so
@@ -569,16 +582,20 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
           dma_one(d, pr, u / 4);
         }
       }
-      soft_x(kk + 1, sc, xa, xh, false);
 #pragma unroll
       for (int m = 24; m < 32; ++m) {
+        if (m == 26) soft_x(kk + 1, sc, xa, xh, false);
         if (m + 3 < 32) va[(m + 3) & 3] = vread(vt, m + 3);
         pv_mfma(va[m & 3], pb[1], m);
+        if (m == 24) {
+          asm volatile("" : "+v"(s_run));  // not ahead of the MFMA
+          soft_s(xa, xh);
+        }
         if (m == 27) dma_one(d, pr, 9);
       }
     };
     // The pass's last block: PV only (its tile is in and synchronised).
-    auto step_last = [&](int kk, const float (&xa)[8], const float (&xh)[8])
+    auto step_last = [&](int kk, float (&xa)[8], float (&xh)[8])
         __attribute__((always_inline)) {
       const uint32_t vt = vbase(kk & (kWideTiles - 1));
       u32x4 va[4], pb[2];
@@ -592,6 +609,7 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
         pv_mfma(va[m & 3], pb[m >> 4], m);
         if (m < 16 && (m & 3) == 1) soft_p(xh, pb[1], m >> 2);
       }
+      soft_s(xa, xh);
     };
     for (int pass = 0;; ++pass) {
 #pragma unroll
@@ -638,9 +656,10 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
         pair_xor32(m_max, lo, hi);
         m_max = fmaxf(lo, hi);
       }
+      const float top = m_max * sx;
       // every load of the pass has landed and every wave is done with the
       // tiles (a second pass, or the next segment, overwrites them)
-      const bool climbed = __builtin_amdgcn_ballot_w64(m_max > m_run + kWideHeadroomLog2) != 0;
+      const bool climbed = __builtin_amdgcn_ballot_w64(top > m_run + kWideHeadroomLog2) != 0;
       if (climbed && lane == 0) s_redo = 1;
       wide_wait_barrier<0>();
       const bool redo = s_redo != 0;
@@ -649,7 +668,7 @@ __global__ __launch_bounds__(256) void mla_wide_kernel(const MlaParams p) {
       if (pass > 0 || !redo) break;
       // scores climbed out of the reference's headroom: again, with the
       // segment's maximum as the reference (no score exceeds it)
-      m_run = m_max;
+      m_run = top;
     }
 
     float lo, hi;
